@@ -100,24 +100,26 @@ struct GemvType {
     const char *gemm_ks_kernel;
     const char *gemm_ks16_kernel;
     const char *gemm_ks4_kernel;
+    const char *gemm_wide_kernel;
     int terms;
     int grid_bytes;
+    double wide_round; /* gemm_wide_toks */
 };
 constexpr GemvType kGemv[] = {
-    {Q38_GGML_Q4_K, "q38_gemv_q8k_q4k", "q38_gemm_q8k_q4k", "q38_gemm_ks_q8k_q4k", "q38_gemm_ks16_q8k_q4k", "q38_gemm_ks4_q8k_q4k", 1, 0},
-    {Q38_GGML_Q5_K, "q38_gemv_q8k_q5k", "q38_gemm_q8k_q5k", "q38_gemm_ks_q8k_q5k", "q38_gemm_ks16_q8k_q5k", "q38_gemm_ks4_q8k_q5k", 1, 0},
-    {Q38_GGML_Q6_K, "q38_gemv_q8k_q6k", "q38_gemm_q8k_q6k", "q38_gemm_ks_q8k_q6k", "q38_gemm_ks16_q8k_q6k", "q38_gemm_ks4_q8k_q6k", 1, 0},
-    {Q38_GGML_Q3_K, "q38_gemv_q8k_q3k", "q38_gemm_q8k_q3k", "q38_gemm_ks_q8k_q3k", "q38_gemm_ks16_q8k_q3k", "q38_gemm_ks4_q8k_q3k", 1, 0},
-    {Q38_GGML_IQ4_XS, "q38_gemv_q8k_iq4xs", "q38_gemm_q8k_iq4xs", "q38_gemm_ks_q8k_iq4xs", "q38_gemm_ks16_q8k_iq4xs", "q38_gemm_ks4_q8k_iq4xs", 1, 0},
-    {Q38_GGML_Q2_K, "q38_gemv_q8k_q2k", "q38_gemm_q8k_q2k", "q38_gemm_ks_q8k_q2k", "q38_gemm_ks16_q8k_q2k", "q38_gemm_ks4_q8k_q2k", 1, 0},
-    {Q38_GGML_IQ4_NL, "q38_gemv_q8k_iq4nl", "q38_gemm_q8k_iq4nl", nullptr, nullptr, nullptr, 8, 0},
-    {Q38_GGML_IQ2_XXS, "q38_gemv_q8k_iq2xxs", "q38_gemm_q8k_iq2xxs", "q38_gemm_ks_q8k_iq2xxs", "q38_gemm_ks16_q8k_iq2xxs", "q38_gemm_ks4_q8k_iq2xxs", 1, 256 * 8},
-    {Q38_GGML_IQ2_XS, "q38_gemv_q8k_iq2xs", "q38_gemm_q8k_iq2xs", "q38_gemm_ks_q8k_iq2xs", "q38_gemm_ks16_q8k_iq2xs", "q38_gemm_ks4_q8k_iq2xs", 1, 512 * 8},
-    {Q38_GGML_IQ2_S, "q38_gemv_q8k_iq2s", "q38_gemm_q8k_iq2s", "q38_gemm_ks_q8k_iq2s", "q38_gemm_ks16_q8k_iq2s", "q38_gemm_ks4_q8k_iq2s", 1, 1024 * 8},
-    {Q38_GGML_IQ3_XXS, "q38_gemv_q8k_iq3xxs", "q38_gemm_q8k_iq3xxs", "q38_gemm_ks_q8k_iq3xxs", "q38_gemm_ks16_q8k_iq3xxs", "q38_gemm_ks4_q8k_iq3xxs", 1, 256 * 4},
-    {Q38_GGML_IQ3_S, "q38_gemv_q8k_iq3s", "q38_gemm_q8k_iq3s", "q38_gemm_ks_q8k_iq3s", "q38_gemm_ks16_q8k_iq3s", "q38_gemm_ks4_q8k_iq3s", 1, 512 * 4},
-    {Q38_GGML_IQ1_S, "q38_gemv_q8k_iq1s", "q38_gemm_q8k_iq1s", "q38_gemm_ks_q8k_iq1s", "q38_gemm_ks16_q8k_iq1s", "q38_gemm_ks4_q8k_iq1s", 1, 2048 * 8},
-    {Q38_GGML_IQ1_M, "q38_gemv_q8k_iq1m", "q38_gemm_q8k_iq1m", "q38_gemm_ks_q8k_iq1m", "q38_gemm_ks16_q8k_iq1m", "q38_gemm_ks4_q8k_iq1m", 1, 2048 * 8},
+    {Q38_GGML_Q4_K, "q38_gemv_q8k_q4k", "q38_gemm_q8k_q4k", "q38_gemm_ks_q8k_q4k", "q38_gemm_ks16_q8k_q4k", "q38_gemm_ks4_q8k_q4k", "q38_gemm_wide_q8k_q4k", 1, 0, 3.0},
+    {Q38_GGML_Q5_K, "q38_gemv_q8k_q5k", "q38_gemm_q8k_q5k", "q38_gemm_ks_q8k_q5k", "q38_gemm_ks16_q8k_q5k", "q38_gemm_ks4_q8k_q5k", "q38_gemm_wide_q8k_q5k", 1, 0, 2.5},
+    {Q38_GGML_Q6_K, "q38_gemv_q8k_q6k", "q38_gemm_q8k_q6k", "q38_gemm_ks_q8k_q6k", "q38_gemm_ks16_q8k_q6k", "q38_gemm_ks4_q8k_q6k", "q38_gemm_wide_q8k_q6k", 1, 0, 2.7},
+    {Q38_GGML_Q3_K, "q38_gemv_q8k_q3k", "q38_gemm_q8k_q3k", "q38_gemm_ks_q8k_q3k", "q38_gemm_ks16_q8k_q3k", "q38_gemm_ks4_q8k_q3k", "q38_gemm_wide_q8k_q3k", 1, 0, 3.2},
+    {Q38_GGML_IQ4_XS, "q38_gemv_q8k_iq4xs", "q38_gemm_q8k_iq4xs", "q38_gemm_ks_q8k_iq4xs", "q38_gemm_ks16_q8k_iq4xs", "q38_gemm_ks4_q8k_iq4xs", "q38_gemm_wide_q8k_iq4xs", 1, 0, 2.4},
+    {Q38_GGML_Q2_K, "q38_gemv_q8k_q2k", "q38_gemm_q8k_q2k", "q38_gemm_ks_q8k_q2k", "q38_gemm_ks16_q8k_q2k", "q38_gemm_ks4_q8k_q2k", "q38_gemm_wide_q8k_q2k", 1, 0, 3.2},
+    {Q38_GGML_IQ4_NL, "q38_gemv_q8k_iq4nl", "q38_gemm_q8k_iq4nl", nullptr, nullptr, nullptr, nullptr, 8, 0, 0.0},
+    {Q38_GGML_IQ2_XXS, "q38_gemv_q8k_iq2xxs", "q38_gemm_q8k_iq2xxs", "q38_gemm_ks_q8k_iq2xxs", "q38_gemm_ks16_q8k_iq2xxs", "q38_gemm_ks4_q8k_iq2xxs", "q38_gemm_wide_q8k_iq2xxs", 1, 256 * 8, 3.4},
+    {Q38_GGML_IQ2_XS, "q38_gemv_q8k_iq2xs", "q38_gemm_q8k_iq2xs", "q38_gemm_ks_q8k_iq2xs", "q38_gemm_ks16_q8k_iq2xs", "q38_gemm_ks4_q8k_iq2xs", "q38_gemm_wide_q8k_iq2xs", 1, 512 * 8, 3.4},
+    {Q38_GGML_IQ2_S, "q38_gemv_q8k_iq2s", "q38_gemm_q8k_iq2s", "q38_gemm_ks_q8k_iq2s", "q38_gemm_ks16_q8k_iq2s", "q38_gemm_ks4_q8k_iq2s", "q38_gemm_wide_q8k_iq2s", 1, 1024 * 8, 3.2},
+    {Q38_GGML_IQ3_XXS, "q38_gemv_q8k_iq3xxs", "q38_gemm_q8k_iq3xxs", "q38_gemm_ks_q8k_iq3xxs", "q38_gemm_ks16_q8k_iq3xxs", "q38_gemm_ks4_q8k_iq3xxs", "q38_gemm_wide_q8k_iq3xxs", 1, 256 * 4, 3.4},
+    {Q38_GGML_IQ3_S, "q38_gemv_q8k_iq3s", "q38_gemm_q8k_iq3s", "q38_gemm_ks_q8k_iq3s", "q38_gemm_ks16_q8k_iq3s", "q38_gemm_ks4_q8k_iq3s", "q38_gemm_wide_q8k_iq3s", 1, 512 * 4, 3.3},
+    {Q38_GGML_IQ1_S, "q38_gemv_q8k_iq1s", "q38_gemm_q8k_iq1s", "q38_gemm_ks_q8k_iq1s", "q38_gemm_ks16_q8k_iq1s", "q38_gemm_ks4_q8k_iq1s", nullptr, 1, 2048 * 8, 0.0},
+    {Q38_GGML_IQ1_M, "q38_gemv_q8k_iq1m", "q38_gemm_q8k_iq1m", "q38_gemm_ks_q8k_iq1m", "q38_gemm_ks16_q8k_iq1m", "q38_gemm_ks4_q8k_iq1m", nullptr, 1, 2048 * 8, 0.0},
 };
 constexpr int kGemvTypes = (int)(sizeof(kGemv) / sizeof(kGemv[0]));
 /* The split-block GEMM's grid: at least this many workgroups (fewer: the
@@ -163,6 +165,7 @@ struct q38_ctx {
     hipFunction_t f_gemm_ks[kGemvTypes] = {};   /* and its split-block form */
     hipFunction_t f_gemm_ks16[kGemvTypes] = {}; /* ... on 16 waves */
     hipFunction_t f_gemm_ks4[kGemvTypes] = {};  /* ... on 4 waves */
+    hipFunction_t f_gemm_wide[kGemvTypes] = {}; /* the 128-token tiles */
     hipFunction_t f_gemv_q8k[kGemvTypes] = {}; /* by kGemv index */
     hipFunction_t f_gemv_f32[3] = {nullptr, nullptr, nullptr}; /* F32, F16, BF16 weights */
     hipFunction_t f_gemm_f32[4] = {nullptr, nullptr, nullptr, nullptr}; /* the same, on the matrix unit */
@@ -473,6 +476,8 @@ int q38_ctx_create(q38_ctx **out, int device, const char *module_dir) {
             Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_ks16[i], ctx->mod_proj, kGemv[i].gemm_ks16_kernel));
         if (kGemv[i].gemm_ks4_kernel != nullptr)
             Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_ks4[i], ctx->mod_proj, kGemv[i].gemm_ks4_kernel));
+        if (kGemv[i].gemm_wide_kernel != nullptr)
+            Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_wide[i], ctx->mod_proj, kGemv[i].gemm_wide_kernel));
     }
     const std::string p_synth = dir + "/synth.hsaco";
     Q38_HIP(hipModuleLoad(&ctx->mod_synth, p_synth.c_str()));
@@ -680,6 +685,7 @@ int q38_kernel_timer_start(q38_ctx *ctx, const char *kernel_name, int max_launch
             if (kGemv[i].gemm_ks_kernel != nullptr && name == kGemv[i].gemm_ks_kernel) f = ctx->f_gemm_ks[i];
             if (kGemv[i].gemm_ks16_kernel != nullptr && name == kGemv[i].gemm_ks16_kernel) f = ctx->f_gemm_ks16[i];
             if (kGemv[i].gemm_ks4_kernel != nullptr && name == kGemv[i].gemm_ks4_kernel) f = ctx->f_gemm_ks4[i];
+            if (kGemv[i].gemm_wide_kernel != nullptr && name == kGemv[i].gemm_wide_kernel) f = ctx->f_gemm_wide[i];
         }
         if (f == nullptr) return fail("unknown kernel %s", kernel_name);
     }
@@ -1946,6 +1952,33 @@ int q38_quantize_q8_k(q38_ctx *ctx, int n_tokens, int width, const float *d_x, v
     return ctx->launch(ctx->f_quantize_q8k, (width / Q38_Q8K_BLOCK + 15) / 16, n_tokens, 1, 256, &a);
 }
 
+/* How many of a call's first tokens take the 128 x 256 tiles (0: none).
+ * One of them runs per CU, so their time goes by whole rounds of cu_count
+ * tiles, while the 128 x 64 tiles, two or three per CU, go by their number;
+ * a small launch adds half a round of its tiles for its start and end.  So as
+ * many full rounds as pay go to the wide tiles and the remaining tokens to
+ * the small ones.  round: a wide round's time in rounds of cu_count small
+ * tiles, measured per format on 17408 x 5120 at 3840 tokens (8 wide rounds,
+ * 31.9 small ones; Q4_K 815 against 1093 us, Q6_K 821 / 1218, Q5_K 865 /
+ * 1393, IQ4_XS 779 / 1301, Q2_K 725 / 890, IQ2_S 1052 / 1314). */
+static int gemm_wide_toks(long row_tiles, int n_tokens, int cu_count, double round) {
+    const long most = ((long)n_tokens + Q38_GEMM_WIDE_TOKENS - 1) / Q38_GEMM_WIDE_TOKENS;
+    if (row_tiles * most > 0x3FFFFFFFL) return 0;
+    double best = 0.0;
+    long best_n = 0;
+    for (long n = 0; n <= most; ++n) {
+        const long rest = std::max(0L, n_tokens - n * Q38_GEMM_WIDE_TOKENS);
+        const long small = row_tiles * ((rest + Q38_GEMM_TOKENS - 1) / Q38_GEMM_TOKENS);
+        const double cost = round * (double)((row_tiles * n + cu_count - 1) / cu_count) +
+                            (small > 0 ? (double)small / cu_count + 0.5 : 0.0);
+        if (n == 0 || cost < best) {
+            best = cost;
+            best_n = n;
+        }
+    }
+    return (int)std::min((long)n_tokens, best_n * Q38_GEMM_WIDE_TOKENS);
+}
+
 /* The projections of one input; d_x non-NULL: the f32 input, quantised into
  * d_q8k as q38_quantize_q8_k does (by the GEMV itself when every matrix
  * stays on it, else by a q38_quantize_q8k launch first). */
@@ -2002,7 +2035,6 @@ static int gemv_q8k_multi(q38_ctx *ctx, int ggml_type, int n_mats, const int *ro
      * 1.4-2x faster).  IQ4_NL, which has only the 128 x 64 form, takes it
      * from Q38_GEMM_IQ4NL_MIN_TOKENS tokens (half as many for 8192+ rows). */
     const int ti = ti_occ;
-    const long tok_tiles = ((long)n_tokens + Q38_GEMM_TOKENS - 1) / Q38_GEMM_TOKENS;
     const long ks_tok_tiles = ((long)n_tokens + Q38_GEMM_KS_TOKENS - 1) / Q38_GEMM_KS_TOKENS;
     bool on_gemv[Q38_GEMV_MAX_MATS] = {}, on_big[Q38_GEMV_MAX_MATS] = {};
     bool any_gemm = false, ks_call = false;
@@ -2030,36 +2062,20 @@ static int gemv_q8k_multi(q38_ctx *ctx, int ggml_type, int n_mats, const int *ro
         if (q38_quantize_q8_k(ctx, n_tokens, width, d_x, const_cast<void *>(d_q8k))) return -1;
         d_x = nullptr;
     }
-    for (int i = 0; i < n_mats; ++i) {
-        if (!on_big[i]) continue;
-        const long row_tiles = ((long)rows[i] + Q38_GEMM_ROWS - 1) / Q38_GEMM_ROWS;
+    /* A launch of the matrix-unit forms over some of the matrices and tokens
+     * tb .. te-1: the matrices with take[i], tile_rows rows a tile */
+    auto gemm_args = [&](const bool *take, long tile_rows, int tb, int te, long &row_tiles) {
         q38_gemv_args g;
         memset(&g, 0, sizeof(g));
-        g.weights[0] = static_cast<const uint8_t *>(d_weights[i]);
-        g.out[0] = d_out[i];
-        g.rows[0] = rows[i];
-        g.n_mats = 1;
-        g.q8k = d_q8k;
-        g.width = width;
-        g.n_tokens = n_tokens;
-        if (ctx->launch(ctx->f_gemm[ti], (unsigned)row_tiles, (unsigned)tok_tiles, 1, 256, &g)) return -1;
-    }
-    if (ks_call) {
-        /* workgroup x serves 32-row tile x - wg_begin[m] of the launch's
-         * matrix m.  Waves per workgroup by workgroups per CU: up to one, 16
-         * waves split the blocks; up to 1.5, 8; beyond, 4 (measured on the
-         * FFN, q|gate and k matrices at 16-256 tokens) */
-        q38_gemv_args g;
-        memset(&g, 0, sizeof(g));
-        long row_tiles = 0;
+        row_tiles = 0;
         int m = 0;
         for (int i = 0; i < n_mats; ++i) {
-            if (rows[i] == 0 || on_big[i]) continue;
+            if (!take[i]) continue;
             g.weights[m] = static_cast<const uint8_t *>(d_weights[i]);
             g.out[m] = d_out[i];
             g.rows[m] = rows[i];
             g.wg_begin[m] = (int32_t)row_tiles;
-            row_tiles += ((long)rows[i] + Q38_GEMM_KS_ROWS - 1) / Q38_GEMM_KS_ROWS;
+            row_tiles += ((long)rows[i] + tile_rows - 1) / tile_rows;
             ++m;
         }
         g.wg_begin[m] = (int32_t)row_tiles;
@@ -2067,16 +2083,66 @@ static int gemv_q8k_multi(q38_ctx *ctx, int ggml_type, int n_mats, const int *ro
         g.q8k = d_q8k;
         g.width = width;
         g.n_tokens = n_tokens;
+        g.tok_begin = tb;
+        g.tok_end = te;
+        return g;
+    };
+    /* The split-block launch of the matrices with take[i]: workgroup x serves
+     * 32-row tile x - wg_begin[m] of the launch's matrix m.  Waves per
+     * workgroup by workgroups per CU: up to one, 16 waves split the blocks; up
+     * to 1.5, 8; beyond, 4 (measured on the FFN, q|gate and k matrices at
+     * 16-256 tokens) */
+    auto launch_ks = [&](const bool *take, int tb, int te) {
+        long row_tiles;
+        q38_gemv_args g = gemm_args(take, Q38_GEMM_KS_ROWS, tb, te, row_tiles);
+        const long toks = ((long)(te - tb) + Q38_GEMM_KS_TOKENS - 1) / Q38_GEMM_KS_TOKENS;
+        const long total = row_tiles * toks;
         hipFunction_t fk = ctx->f_gemm_ks[ti];
         int waves = Q38_GEMM_KS_WAVES;
-        if (ks_total <= (long)ctx->cu_count && ctx->f_gemm_ks16[ti] != nullptr) {
+        if (total <= (long)ctx->cu_count && ctx->f_gemm_ks16[ti] != nullptr) {
             fk = ctx->f_gemm_ks16[ti];
             waves = Q38_GEMM_KS_WAVES_WIDE;
-        } else if (2 * ks_total > 3L * ctx->cu_count && ctx->f_gemm_ks4[ti] != nullptr) {
+        } else if (2 * total > 3L * ctx->cu_count && ctx->f_gemm_ks4[ti] != nullptr) {
             fk = ctx->f_gemm_ks4[ti];
             waves = Q38_GEMM_KS_WAVES_NARROW;
         }
-        if (ctx->launch(fk, (unsigned)row_tiles, (unsigned)ks_tok_tiles, 1, 64 * waves, &g)) return -1;
+        return ctx->launch(fk, (unsigned)row_tiles, (unsigned)toks, 1, 64 * waves, &g);
+    };
+    /* The tiled matrices' tokens, the first wide_toks of them on the 128 x 256
+     * tiles (gemm_wide_toks) and the rest, per matrix, on the split-block form
+     * or the 128 x 64 tiles by the rule above */
+    long wide_row_tiles = 0;
+    for (int i = 0; i < n_mats; ++i)
+        if (on_big[i]) wide_row_tiles += ((long)rows[i] + Q38_GEMM_ROWS - 1) / Q38_GEMM_ROWS;
+    const int wide_toks = ctx->f_gemm_wide[ti] != nullptr && wide_row_tiles > 0
+                              ? gemm_wide_toks(wide_row_tiles, n_tokens, ctx->cu_count, kGemv[ti].wide_round)
+                              : 0;
+    if (wide_toks > 0) {
+        long row_tiles;
+        q38_gemv_args g = gemm_args(on_big, Q38_GEMM_ROWS, 0, wide_toks, row_tiles);
+        const long tiles = row_tiles * (((long)wide_toks + Q38_GEMM_WIDE_TOKENS - 1) / Q38_GEMM_WIDE_TOKENS);
+        if (ctx->launch(ctx->f_gemm_wide[ti], (unsigned)((tiles + 7) / 8 * 8), 1, 1, 512, &g)) return -1;
+    }
+    for (int i = 0; i < n_mats && wide_toks < n_tokens; ++i) {
+        if (!on_big[i]) continue;
+        bool only[Q38_GEMV_MAX_MATS] = {};
+        only[i] = true;
+        const int rest = n_tokens - wide_toks;
+        const long ks_tiles = ((long)rows[i] + Q38_GEMM_KS_ROWS - 1) / Q38_GEMM_KS_ROWS *
+                              (((long)rest + Q38_GEMM_KS_TOKENS - 1) / Q38_GEMM_KS_TOKENS);
+        if (ctx->f_gemm_ks[ti] != nullptr && ks_tiles <= kGemmKsMaxPerCu * (long)ctx->cu_count) {
+            if (launch_ks(only, wide_toks, n_tokens)) return -1;
+            continue;
+        }
+        long row_tiles;
+        q38_gemv_args g = gemm_args(only, Q38_GEMM_ROWS, wide_toks, n_tokens, row_tiles);
+        const long toks = ((long)rest + Q38_GEMM_TOKENS - 1) / Q38_GEMM_TOKENS;
+        if (ctx->launch(ctx->f_gemm[ti], (unsigned)row_tiles, (unsigned)toks, 1, 256, &g)) return -1;
+    }
+    if (ks_call) {
+        bool others[Q38_GEMV_MAX_MATS] = {};
+        for (int i = 0; i < n_mats; ++i) others[i] = rows[i] > 0 && !on_big[i];
+        if (launch_ks(others, 0, n_tokens)) return -1;
     }
 
     /* The GEMV over the other matrices, in one launch.  Tokens per pass: as

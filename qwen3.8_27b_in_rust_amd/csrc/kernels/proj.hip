@@ -1242,6 +1242,76 @@ Q38_DEV uint32_t fold_weights(uint32_t q, int sc) {
     }
 }
 
+/* The byte planes of the lane's 16 scaled weights of k step st: bh alone,
+ * bh and bl, or (Q5_K) bh, bl and bx; bm the bytes of the second sum. */
+template <int TYPE>
+Q38_DEV void gemm_step_planes(const Unit<TYPE> &u, const UnitScales<TYPE> &s, uint32_t hm, const uint8_t *grid, int st,
+                              i32x4 &bh, i32x4 &bl, i32x4 &bx, i32x4 &bm) {
+    auto word = [&](int k) { return kGemmHalfUnit<TYPE> ? u.w[k] : (u.w[k] & ~hm) | (u.w[k + 4] & hm); };
+    if constexpr (TYPE == Q38_GGML_Q4_K) {
+        /* w = sc q with sc = 8 sh + sl: the planes q sh and q sl
+         * (at most 15 x 7 = 105 per byte) are packed 16-bit
+         * products of the quant bytes, no carry between bytes */
+        const unsigned short sh = (unsigned short)(s.sc[st] >> 3), sl = (unsigned short)(s.sc[st] & 7);
+        const u16x2 SH = {sh, sh}, SL = {sl, sl};
+        const int c = st >> 1, nib = st & 1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const u16x2 q = __builtin_bit_cast(u16x2, (word(4 + 8 * c + j) >> (4 * nib)) & 0x0F0F0F0Fu);
+            bh[j] = __builtin_bit_cast(int, q * SH);
+            bl[j] = __builtin_bit_cast(int, q * SL);
+            bm[j] = s.mn[st] * 0x01010101;
+        }
+    } else if constexpr (TYPE == Q38_GGML_Q5_K) {
+        /* w = sc q, q <= 31: three planes of sc = 16 s2 + 4 s1 +
+         * s0 (each at most 3, q s <= 93 per byte) */
+        const unsigned short s2 = (unsigned short)(s.sc[st] >> 4), s1 = (unsigned short)((s.sc[st] >> 2) & 3),
+                             s0 = (unsigned short)(s.sc[st] & 3);
+        const u16x2 S2 = {s2, s2}, S1 = {s1, s1}, S0 = {s0, s0};
+        const int c = st >> 1, nib = st & 1;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t qv = ((word(12 + 8 * c + j) >> (4 * nib)) & 0x0F0F0F0Fu) |
+                                (((word(4 + j) >> st) & 0x01010101u) << 4);
+            const u16x2 q = __builtin_bit_cast(u16x2, qv);
+            bh[j] = __builtin_bit_cast(int, q * S2);
+            bl[j] = __builtin_bit_cast(int, q * S1);
+            bx[j] = __builtin_bit_cast(int, q * S0);
+            bm[j] = s.mn[st] * 0x01010101;
+        }
+    } else if constexpr (TYPE == Q38_GGML_Q6_K) {
+        const int sc = (int)(((uint32_t)s.sc[2 * st] & ~hm) | ((uint32_t)s.sc[2 * st + 1] & hm));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int hf = st >> 2, kq = st & 3;
+            const uint32_t ql = word(16 * hf + 8 * (kq & 1) + j);
+            const uint32_t qh = word(32 + 8 * hf + j);
+            const uint32_t q = ((ql >> (4 * (kq >> 1))) & 0x0F0F0F0Fu) | (((qh >> (2 * kq)) & 0x03030303u) << 4);
+            uint32_t hi, lo;
+            split_weights(q, sc, (short)32, hi, lo);
+            bh[j] = (int)hi;
+            bl[j] = (int)lo;
+        }
+    } else {
+        uint32_t q[4], second[4];
+        int sc;
+        short off;
+        gemm_step_bytes<TYPE>(u, s, st, hm, grid, q, sc, off, second);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if constexpr (kGemmPlanes<TYPE> == 1) {
+                bh[j] = (int)fold_weights<TYPE>(q[j], sc);
+            } else {
+                uint32_t hi, lo;
+                split_weights(q[j], sc, off, hi, lo);
+                bh[j] = (int)hi;
+                bl[j] = (int)lo;
+            }
+            bm[j] = (int)second[j];
+        }
+    }
+}
+
 /* One block's f32 terms for a tile of 32 tokens x 32 rows (the lane's 16
  * outputs: row l % 32, tokens 8J + 4(l/32) + i for element 4J + i): the
  * integer sums on the matrix unit, then the reference's f32 block term.
@@ -1251,73 +1321,11 @@ Q38_DEV uint32_t fold_weights(uint32_t q, int sc) {
 template <int TYPE, typename AOf, typename AsOf, typename Sink>
 Q38_DEV void gemm_tile_terms(const Unit<TYPE> &u, const UnitScales<TYPE> &s, uint32_t hm, const uint8_t *grid,
                              AOf A_of, AsOf as_of, Sink sink) {
-    auto word = [&](int k) { return kGemmHalfUnit<TYPE> ? u.w[k] : (u.w[k] & ~hm) | (u.w[k + 4] & hm); };
     i32x16 wsum = i32x16{}, lsum = i32x16{}, xsum = i32x16{}, msum = i32x16{};
 #pragma unroll
     for (int st = 0; st < 8; ++st) {
         i32x4 bh, bl, bx, bm;
-        if constexpr (TYPE == Q38_GGML_Q4_K) {
-            /* w = sc q with sc = 8 sh + sl: the planes q sh and q sl
-             * (at most 15 x 7 = 105 per byte) are packed 16-bit
-             * products of the quant bytes, no carry between bytes */
-            const unsigned short sh = (unsigned short)(s.sc[st] >> 3), sl = (unsigned short)(s.sc[st] & 7);
-            const u16x2 SH = {sh, sh}, SL = {sl, sl};
-            const int c = st >> 1, nib = st & 1;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const u16x2 q = __builtin_bit_cast(u16x2, (word(4 + 8 * c + j) >> (4 * nib)) & 0x0F0F0F0Fu);
-                bh[j] = __builtin_bit_cast(int, q * SH);
-                bl[j] = __builtin_bit_cast(int, q * SL);
-                bm[j] = s.mn[st] * 0x01010101;
-            }
-        } else if constexpr (TYPE == Q38_GGML_Q5_K) {
-            /* w = sc q, q <= 31: three planes of sc = 16 s2 + 4 s1 +
-             * s0 (each at most 3, q s <= 93 per byte) */
-            const unsigned short s2 = (unsigned short)(s.sc[st] >> 4), s1 = (unsigned short)((s.sc[st] >> 2) & 3),
-                                 s0 = (unsigned short)(s.sc[st] & 3);
-            const u16x2 S2 = {s2, s2}, S1 = {s1, s1}, S0 = {s0, s0};
-            const int c = st >> 1, nib = st & 1;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t qv = ((word(12 + 8 * c + j) >> (4 * nib)) & 0x0F0F0F0Fu) |
-                                    (((word(4 + j) >> st) & 0x01010101u) << 4);
-                const u16x2 q = __builtin_bit_cast(u16x2, qv);
-                bh[j] = __builtin_bit_cast(int, q * S2);
-                bl[j] = __builtin_bit_cast(int, q * S1);
-                bx[j] = __builtin_bit_cast(int, q * S0);
-                bm[j] = s.mn[st] * 0x01010101;
-            }
-        } else if constexpr (TYPE == Q38_GGML_Q6_K) {
-            const int sc = (int)(((uint32_t)s.sc[2 * st] & ~hm) | ((uint32_t)s.sc[2 * st + 1] & hm));
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int hf = st >> 2, kq = st & 3;
-                const uint32_t ql = word(16 * hf + 8 * (kq & 1) + j);
-                const uint32_t qh = word(32 + 8 * hf + j);
-                const uint32_t q = ((ql >> (4 * (kq >> 1))) & 0x0F0F0F0Fu) | (((qh >> (2 * kq)) & 0x03030303u) << 4);
-                uint32_t hi, lo;
-                split_weights(q, sc, (short)32, hi, lo);
-                bh[j] = (int)hi;
-                bl[j] = (int)lo;
-            }
-        } else {
-            uint32_t q[4], second[4];
-            int sc;
-            short off;
-            gemm_step_bytes<TYPE>(u, s, st, hm, grid, q, sc, off, second);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if constexpr (kGemmPlanes<TYPE> == 1) {
-                    bh[j] = (int)fold_weights<TYPE>(q[j], sc);
-                } else {
-                    uint32_t hi, lo;
-                    split_weights(q[j], sc, off, hi, lo);
-                    bh[j] = (int)hi;
-                    bl[j] = (int)lo;
-                }
-                bm[j] = (int)second[j];
-            }
-        }
+        gemm_step_planes<TYPE>(u, s, hm, grid, st, bh, bl, bx, bm);
         const i32x4 A = A_of(st);
         wsum = mfma_i8(A, bh, wsum);
         if constexpr (kGemmPlanes<TYPE> >= 2) lsum = mfma_i8(A, bl, lsum);
@@ -1369,7 +1377,7 @@ Q38_DEV void gemm_q8k(const q38_gemv_args &a) {
     const int rows = a.rows[0];
     const int row = blockIdx.x * kGemmRows + wave * 32 + (lane & 31);
     const int rowc = min(row, rows - 1);
-    const int t0 = blockIdx.y * kGemmTokens;
+    const int t0 = a.tok_begin + blockIdx.y * kGemmTokens;
     const int T = a.n_tokens;
     const int8_t *quants = static_cast<const int8_t *>(a.q8k);
     const int16_t *sums = reinterpret_cast<const int16_t *>(quants + (size_t)T * width);
@@ -1418,6 +1426,478 @@ Q38_DEV void gemm_q8k(const q38_gemv_args &a) {
 }
 
 
+/* Long prompts: a workgroup of 8 waves owns 128 rows x NT tokens (256 or 128),
+ * wave w the 16 rows 16 w .. + 15 and every token, as 16 x 16 tiles
+ * (v_mfma_i32_16x16x64_i8).  A SIMD issues one vector or matrix instruction
+ * about every 4 cycles, whichever of its waves it comes from, and the 128 x 64
+ * tiles above spent 1.7 times the matrix unit's time issuing conversions and
+ * block terms (17408 x 5120 Q4_K, 3001 tokens).  So this form is built to issue
+ * fewer of them:
+ *  - a block's weights become byte planes once for NT tokens, each lane
+ *    reading and converting only its own 64 of the 256 (lane l: row l % 16;
+ *    of the block, k half hb = (l / 16) % 2, and of each 32 values the 16 of
+ *    half h = l / 32);
+ *  - the minimum sum_j m_j bsum_j is ONE f16 step over the activations' 16
+ *    group sums (|sum of 16 quants| <= 2032 and |m_j| <= 63: exact in f16,
+ *    the sum below 2^21 exact in f32), already a float;
+ *  - the products d a_scale and dmin a_scale of two token groups are one f32
+ *    step of four 16 x 16 x 1 blocks (a product and + 0: the rounding of one
+ *    multiply), 1 instruction for 16;
+ *  - the next block's activations go to the other LDS buffer by
+ *    direct-to-LDS loads, its weights to registers, while this one computes:
+ *    one barrier per block.  Rows of 256 bytes hold the 16 bytes of (hb, p, h)
+ *    of token t at chunk (4 p + 2 hb + h) ^ (t % 16): no padding (the loads fill
+ *    whole KiB), and the 16 lanes that a 16-byte LDS read serves together (8
+ *    of one k quarter, the other 8 tokens of the next) meet distinct banks --
+ *    with hb in the chunk's top bit they met in pairs.
+ * Measured: 17408 x 5120 at 3840 tokens Q4_K 815 us against 1093 on the 128 x
+ * 64 tiles (840 against 626 TOPS), Q6_K 821 / 1218, Q5_K 865 / 1393, Q3_K 780
+ * / 961, Q2_K 725 / 890, IQ4_XS 779 / 1301, IQ2_S 1052 / 1314, IQ3_S 1150 /
+ * 1406.  Bound now by what the two waves of a SIMD issue: matrix unit busy
+ * 47% of the cycles, vector issue 51%, 15% of them at once, at the 1.9 GHz
+ * the part keeps under this load.  Measured and not kept: 32 x 32 tiles (half
+ * the matrix instructions, no room for two tiles' accumulators: 5-25%
+ * slower), a higher priority for one wave of each SIMD (no change).
+ * A launch holds up to Q38_GEMV_MAX_MATS matrices of one input (row tiles
+ * wg_begin[m] ..), its tiles in bands of 8 row tiles walked along the tokens,
+ * a contiguous stretch of them per XCD, so that the 32 workgroups an XCD runs
+ * at once share 8 row tiles' weights and 4 token tiles in its L2. */
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr int kWideThreads = 512;
+
+/* Formats with a minimum: a second sum, over the activations' groups, and a
+ * second scale */
+template <int TYPE> constexpr bool kHasMin =
+    TYPE == Q38_GGML_Q2_K || TYPE == Q38_GGML_Q4_K || TYPE == Q38_GGML_Q5_K;
+
+/* A lane's part of a block: 64 weights (values 128 hb + 32 p + 16 h .. + 15 for
+ * p = 0..3) and their scales.  The formats of the largest files load just
+ * that; the lattice formats load the block and pick (Whole). */
+template <int TYPE> struct Part {
+    Unit<TYPE> u;
+};
+template <> struct Part<Q38_GGML_Q4_K> { u32x4 head, q[2]; };
+template <> struct Part<Q38_GGML_Q5_K> { u32x4 head, high, q[2]; };
+template <> struct Part<Q38_GGML_Q6_K> { u32x4 ql[2], qh, sc; uint32_t dh; };
+template <> struct Part<Q38_GGML_Q2_K> { u32x4 sc, q; uint32_t dd; };
+template <> struct Part<Q38_GGML_Q3_K> { u32x4 high, q, sc; uint32_t dh; };
+template <> struct Part<Q38_GGML_IQ4_XS> { u32x4 q[4]; uint32_t w0, w1; };
+template <int TYPE> constexpr bool kWholePart =
+    !(TYPE == Q38_GGML_Q4_K || TYPE == Q38_GGML_Q5_K || TYPE == Q38_GGML_Q6_K || TYPE == Q38_GGML_Q2_K ||
+      TYPE == Q38_GGML_Q3_K || TYPE == Q38_GGML_IQ4_XS);
+
+/* 16 bytes at a dword boundary */
+Q38_DEV u32x4 load16_4aligned(const uint8_t *p) {
+    u32x4 v;
+    __builtin_memcpy(&v, reinterpret_cast<const uint32_t *>(p), 16);
+    return v;
+}
+
+template <int TYPE>
+Q38_DEV void load_part(const uint8_t *weights, size_t g, int hb, int h, Part<TYPE> &u) {
+    const uint8_t *blk = weights + g * KQuant<TYPE>::bytes;
+    if constexpr (TYPE == Q38_GGML_Q4_K || TYPE == Q38_GGML_Q5_K) {
+        u.head = *reinterpret_cast<const u32x4 *>(blk);
+        if constexpr (TYPE == Q38_GGML_Q5_K) u.high = *reinterpret_cast<const u32x4 *>(blk + 16 + 16 * h);
+        const uint8_t *qs = blk + (TYPE == Q38_GGML_Q5_K ? 48 : 16) + 64 * hb + 16 * h;
+        u.q[0] = *reinterpret_cast<const u32x4 *>(qs);
+        u.q[1] = *reinterpret_cast<const u32x4 *>(qs + 32);
+    } else if constexpr (TYPE == Q38_GGML_Q6_K) {
+        const uint32_t o = (uint32_t)((g * 210) & 3); /* 0 or 2 */
+        u.ql[0] = load16_2aligned(blk, o, 64 * hb + 16 * h, false);
+        u.ql[1] = load16_2aligned(blk, o, 64 * hb + 16 * h + 32, false);
+        u.qh = load16_2aligned(blk, o, 128 + 32 * hb + 16 * h, false);
+        u.sc = load16_2aligned(blk, o, 192, true);
+        u.dh = *reinterpret_cast<const uint16_t *>(blk + 208);
+    } else if constexpr (TYPE == Q38_GGML_Q2_K) {
+        u.sc = load16_4aligned(blk);
+        u.q = load16_4aligned(blk + 16 + 32 * hb + 16 * h);
+        u.dd = *reinterpret_cast<const uint32_t *>(blk + 80);
+    } else if constexpr (TYPE == Q38_GGML_Q3_K) {
+        /* 32 mask bytes, 64 quant bytes, 12 scale bytes, the f16 scale: the
+         * 16 bytes from 92 on hold the scale bytes in their last 12 */
+        const uint32_t o = (uint32_t)((g * 110) & 3); /* 0 or 2 */
+        u.high = load16_2aligned(blk, o, 16 * h, false);
+        u.q = load16_2aligned(blk, o, 32 + 32 * hb + 16 * h, false);
+        u.sc = load16_2aligned(blk, o, 92, true);
+        u.dh = *reinterpret_cast<const uint16_t *>(blk + 108);
+    } else if constexpr (TYPE == Q38_GGML_IQ4_XS) {
+        u.w0 = *reinterpret_cast<const uint32_t *>(blk);
+        u.w1 = *reinterpret_cast<const uint32_t *>(blk + 4);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) u.q[p] = load16_4aligned(blk + 8 + 64 * hb + 16 * p);
+    } else {
+        load_unit<TYPE>(weights, g, u.u);
+    }
+}
+
+/* The part's byte planes (step p: values 128 hb + 32 p + 16 h ..), the
+ * multipliers of the 8 group sums 8 hb .. 8 hb + 7 (zero in
+ * the lanes h = 1, whose k quarters are beyond the 16 groups) and the block's
+ * f32 scales.  hbm and hm: lane masks of hb and h (lane_half_mask). */
+template <int TYPE>
+Q38_DEV void part_planes(const Part<TYPE> &u, uint32_t hbm, uint32_t hm, const uint8_t *grid, i32x4 (&bh)[4],
+                         i32x4 (&bl)[4], f16x8 &mults, float &d, float &dmin) {
+    auto pick = [&](uint32_t a0, uint32_t a1) { return (a0 & ~hbm) | (a1 & hbm); };
+    /* byte p of w in both 16-bit halves */
+    auto splat16 = [&](uint32_t w, int p) { return __builtin_amdgcn_perm(0u, w, 0x0c000c00u | (uint32_t)(p | (p << 16))); };
+    int mn[4] = {0, 0, 0, 0}; /* multipliers, one per pair of groups, or */
+    int mn8[8] = {};          /* one per group (Q2_K) */
+    dmin = 0.0f;
+    if constexpr (TYPE == Q38_GGML_Q4_K || TYPE == Q38_GGML_Q5_K) {
+        /* scale_min_k4 on 4 bytes at once: sub-blocks 0-3 or 4-7 */
+        const uint32_t s0 = u.head.y, s1 = u.head.z, s2 = u.head.w;
+        const uint32_t sc = pick(s0 & 0x3F3F3F3Fu, (s2 & 0x0F0F0F0Fu) | ((s0 >> 2) & 0x30303030u));
+        const uint32_t mw = pick(s1 & 0x3F3F3F3Fu, ((s2 >> 4) & 0x0F0F0F0Fu) | ((s1 >> 2) & 0x30303030u));
+#pragma unroll
+        for (int p = 0; p < 4; ++p) mn[p] = (int)((mw >> (8 * p)) & 255u);
+        if constexpr (TYPE == Q38_GGML_Q4_K) {
+            const uint32_t sh = (sc >> 3) & 0x07070707u, sl = sc & 0x07070707u;
+#pragma unroll
+            for (int p = 0; p < 4; ++p) {
+                const u16x2 SH = __builtin_bit_cast(u16x2, splat16(sh, p)), SL = __builtin_bit_cast(u16x2, splat16(sl, p));
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const u16x2 q = __builtin_bit_cast(u16x2, (u.q[p >> 1][j] >> (4 * (p & 1))) & 0x0F0F0F0Fu);
+                    bh[p][j] = __builtin_bit_cast(int, q * SH);
+                    bl[p][j] = __builtin_bit_cast(int, q * SL);
+                }
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t hi4 = pick(u.high[j], u.high[j] >> 4); /* bit p of a byte: sub-block 4 hb + p */
+#pragma unroll
+                for (int p = 0; p < 4; ++p) {
+                    const uint32_t q = ((u.q[p >> 1][j] >> (4 * (p & 1))) & 0x0F0F0F0Fu) | (((hi4 >> p) & 0x01010101u) << 4);
+                    uint32_t hi, lo;
+                    split_weights(q, (int)((sc >> (8 * p)) & 255u), (short)0, hi, lo);
+                    bh[p][j] = (int)hi;
+                    bl[p][j] = (int)lo;
+                }
+            }
+        }
+        d = q38_f16(u.head.x);
+        dmin = q38_f16(u.head.x >> 16);
+    } else if constexpr (TYPE == Q38_GGML_Q6_K) {
+        /* the 8 scales of groups 8 hb ..; step p's group is 2 p + h */
+        const uint32_t e0 = pick(u.sc.x, u.sc.z), e1 = pick(u.sc.y, u.sc.w);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const uint32_t w = p < 2 ? e0 : e1;
+            const int s0 = (int)(int8_t)((w >> (16 * (p & 1))) & 255u), s1 = (int)(int8_t)((w >> (16 * (p & 1) + 8)) & 255u);
+            const int sc = (int)(((uint32_t)s0 & ~hm) | ((uint32_t)s1 & hm));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t q = ((u.ql[p & 1][j] >> (4 * (p >> 1))) & 0x0F0F0F0Fu) |
+                                   (((u.qh[j] >> (2 * p)) & 0x03030303u) << 4);
+                uint32_t hi, lo;
+                split_weights(q, sc, (short)32, hi, lo);
+                bh[p][j] = (int)hi;
+                bl[p][j] = (int)lo;
+            }
+        }
+        d = q38_f16(u.dh);
+    } else if constexpr (TYPE == Q38_GGML_Q2_K) {
+        const uint32_t e[2] = {pick(u.sc.x, u.sc.z), pick(u.sc.y, u.sc.w)}; /* scale bytes of groups 8 hb .. */
+#pragma unroll
+        for (int k = 0; k < 8; ++k) mn8[k] = (int)((e[k >> 2] >> (8 * (k & 3) + 4)) & 15u);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const uint32_t w = e[p >> 1] >> (16 * (p & 1));
+            const int sc = (int)((((w & ~hm) | ((w >> 8) & hm))) & 15u);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) bh[p][j] = (int)fold_weights<TYPE>((u.q[j] >> (2 * p)) & 0x03030303u, sc);
+        }
+        d = q38_f16(u.dd);
+        dmin = q38_f16(u.dd >> 16);
+    } else if constexpr (TYPE == Q38_GGML_Q3_K) {
+        /* group g = 8 hb + 2 p + h: low nibble (hb = 0) or high nibble (1)
+         * of scale byte 2 p + h, high 2 bits from byte 8 + g % 4 at 2 (g / 4)
+         * (unpack_q3_scales); the scale bytes are words 1..3 of u.sc */
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const uint32_t lw = (p < 2 ? u.sc.y : u.sc.z) >> (16 * (p & 1));
+            const uint32_t low = pick((lw & ~hm) | ((lw >> 8) & hm), ((lw >> 4) & ~hm) | ((lw >> 12) & hm)) & 15u;
+            const uint32_t hw = u.sc.w >> (16 * (p & 1) + 2 * (p >> 1));
+            const uint32_t hx = (hw & ~hm) | ((hw >> 8) & hm);
+            const int sc = (int)(low | ((pick(hx, hx >> 4) & 3u) << 4)) - 32;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t q = ((u.q[j] >> (2 * p)) & 0x03030303u) |
+                                   ((pick(u.high[j] >> p, u.high[j] >> (4 + p)) & 0x01010101u) << 2);
+                bh[p][j] = (int)fold_weights<TYPE>(q, sc);
+            }
+        }
+        d = q38_f16(u.dh);
+    } else if constexpr (TYPE == Q38_GGML_IQ4_XS) {
+        const uint32_t sl = pick(u.w1, u.w1 >> 16), sh = pick(u.w0 >> 16, u.w0 >> 24); /* of groups 4 hb .. */
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int sc = (int)(((sl >> (4 * p)) & 15u) | (((sh >> (2 * p)) & 3u) << 4)) - 32;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t x = u.q[p][j];
+                const uint32_t q = q38_iq4_lookup(((x & ~hm) | ((x >> 4) & hm)) & 0x0F0F0F0Fu) ^ 0x80808080u;
+                uint32_t hi, lo;
+                split_weights(q, sc, (short)128, hi, lo);
+                bh[p][j] = (int)hi;
+                bl[p][j] = (int)lo;
+            }
+        }
+        d = q38_f16(u.w0);
+    } else {
+        UnitScales<TYPE> s;
+        unit_scales<TYPE>(u.u, s);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            i32x4 h0, l0, x0, m0, h1, l1, x1, m1;
+            gemm_step_planes<TYPE>(u.u, s, hm, grid, p, h0, l0, x0, m0);
+            gemm_step_planes<TYPE>(u.u, s, hm, grid, 4 + p, h1, l1, x1, m1);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                bh[p][j] = (int)pick((uint32_t)h0[j], (uint32_t)h1[j]);
+                if constexpr (kGemmPlanes<TYPE> >= 2) bl[p][j] = (int)pick((uint32_t)l0[j], (uint32_t)l1[j]);
+            }
+        }
+        d = s.d;
+    }
+    if constexpr (kHasMin<TYPE>) {
+        u32x4 m;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float m0 = (float)(TYPE == Q38_GGML_Q2_K ? mn8[2 * k] : mn[k]);
+            const float m1 = (float)(TYPE == Q38_GGML_Q2_K ? mn8[2 * k + 1] : mn[k]);
+            m[k] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(m0, m1)) & ~hm; /* whole numbers: exact */
+        }
+        mults = __builtin_bit_cast(f16x8, m);
+    }
+}
+
+template <int TYPE, int NT>
+Q38_DEV void gemm_wide_q8k(const q38_gemv_args &a) {
+    constexpr int kTiles = NT / 16; /* 16 x 16 tiles of a wave */
+    static_assert(TYPE != Q38_GGML_IQ1_S && TYPE != Q38_GGML_IQ1_M, "IQ1 takes the 128 x 64 tiles");
+    __shared__ __align__(16) int8_t act[2][NT][256];
+    __shared__ __align__(16) float ascale[2][NT];
+    __shared__ __align__(16) _Float16 gsum[2][kHasMin<TYPE> ? NT : 1][16];
+    constexpr int kGridBytes = IqGrid<TYPE>::bytes;
+    __shared__ __align__(16) uint8_t grid[kGridBytes > 0 ? kGridBytes : 16];
+    const int tid = threadIdx.x;
+    if constexpr (kGridBytes > 0) {
+        const u32x4 *src = static_cast<const u32x4 *>(iq_grid_table<TYPE>());
+        for (int i = tid; i < kGridBytes / 16; i += kWideThreads) reinterpret_cast<u32x4 *>(grid)[i] = src[i];
+    }
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c16 = lane & 15; /* activation row (token) and output column (weight row) of the tiles */
+    const int q = lane >> 4;   /* k quarter of a 64-value step */
+    const int hb = q & 1, h = q >> 1;
+    const uint32_t hbm = lane_half_mask(hb), hm = lane_half_mask(h);
+    const int width = a.width;
+    const int B = width / Q38_Q8K_BLOCK;
+    const int T = a.n_tokens;
+
+    /* workgroup -> tile: tiles numbered in bands of 8 row tiles, XCD x takes
+     * numbers x * per .. x * per + per - 1 */
+    const int row_tiles = a.wg_begin[a.n_mats];
+    const int tok_end = a.tok_end;
+    const int tok_tiles = (tok_end - a.tok_begin + NT - 1) / NT;
+    const int n_tiles = row_tiles * tok_tiles;
+    const int per = (n_tiles + 7) / 8;
+    const int L = ((int)blockIdx.x & 7) * per + ((int)blockIdx.x >> 3);
+    if (L >= n_tiles || ((int)blockIdx.x >> 3) >= per) return; /* the same for the whole workgroup */
+    const int band = L / (8 * tok_tiles);
+    const int in_band = L - band * 8 * tok_tiles;
+    const int band_rows = min(8, row_tiles - 8 * band);
+    const int tt0 = in_band / band_rows;
+    const int rt = 8 * band + in_band - tt0 * band_rows;
+    int mat = 0;
+#pragma unroll
+    for (int i = 1; i < Q38_GEMV_MAX_MATS; ++i) mat += (i < a.n_mats && rt >= a.wg_begin[i]) ? 1 : 0;
+    const uint8_t *weights = a.weights[mat];
+    float *out = a.out[mat];
+    const int rows = a.rows[mat];
+    const int row = (rt - a.wg_begin[mat]) * kGemmRows + wave * 16 + c16;
+    const size_t unit0 = (size_t)min(row, rows - 1) * B;
+    const int t0 = a.tok_begin + tt0 * NT;
+    const int8_t *quants = static_cast<const int8_t *>(a.q8k);
+    const int16_t *sums = reinterpret_cast<const int16_t *>(quants + (size_t)T * width);
+    const float *scales = reinterpret_cast<const float *>(sums + (size_t)T * B * 16);
+
+    /* direct-to-LDS: wave w moves pieces w, w + 8, ... of 1 KiB (4 tokens);
+     * lane l's 16 bytes land at 16 l of the piece: token l / 16, chunk l % 16
+     * of the swizzled row; tokens past the prompt read the last one */
+    constexpr int kMyPieces = NT / 4 / 8;
+    uint32_t src_off[kMyPieces];
+#pragma unroll
+    for (int i = 0; i < kMyPieces; ++i) {
+        const int t = 4 * (wave + 8 * i) + q;
+        const uint32_t x = (uint32_t)(c16 ^ (t & 15)); /* 4 p + 2 hb + h of the chunk */
+        src_off[i] = (uint32_t)(min(t0 + t, T - 1) - t0) * (uint32_t)width + 16u * (8 * ((x >> 1) & 1) + 2 * (x >> 2) + (x & 1));
+    }
+    const int8_t *q_base = quants + (size_t)t0 * width;
+    auto fetch_acts = [&](int b, int buf) {
+#pragma unroll
+        for (int i = 0; i < kMyPieces; ++i) {
+            const uint32_t lds =
+                (uint32_t)(size_t)(__attribute__((address_space(3))) int8_t *)&act[buf][4 * (wave + 8 * i)][0];
+            /* one wait state between the M0 write and the load that reads it */
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(src_off[i]),
+                         "s"(q_base + b * 256)
+                         : "memory");
+        }
+    };
+    /* a thread's share of the scales (token tid) and group sums (8 of token
+     * tid / 2) */
+    const size_t sc_at = (size_t)min(t0 + (tid & (NT - 1)), T - 1) * B;
+    const size_t gs_at = (size_t)min(t0 + (tid >> 1) % NT, T - 1) * B;
+    float my_scale;
+    u32x4 my_sums = {};
+    Part<TYPE> u;
+    auto fetch_regs = [&](int b) {
+        load_part<TYPE>(weights, unit0 + b, hb, h, u);
+        my_scale = scales[sc_at + b];
+        if constexpr (kHasMin<TYPE>)
+            my_sums = *reinterpret_cast<const u32x4 *>(sums + (gs_at + b) * 16 + 8 * (tid & 1));
+    };
+
+    f32x4 total[kTiles]; /* tile i: tokens 16 i .. of the wave's 16 rows */
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i) total[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    fetch_acts(0, 0);
+    fetch_regs(0);
+    for (int b = 0; b < B; ++b) {
+        const int buf = b & 1;
+        if (tid < NT) ascale[buf][tid] = my_scale;
+        if constexpr (kHasMin<TYPE>) {
+            f16x8 g8;
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                g8[k] = (_Float16)(float)(int)(int16_t)((my_sums[k >> 1] >> (16 * (k & 1))) & 0xffffu);
+            if (tid < 2 * NT) *reinterpret_cast<f16x8 *>(&gsum[buf][tid >> 1][8 * (tid & 1)]) = g8;
+        }
+        /* this block's activations have landed (every wave's share), and every
+         * wave is done with the other buffer */
+        q38_barrier_vm<0>();
+        i32x4 bh[4], bl[4];
+        f16x8 mults = {};
+        float d, dmin;
+        part_planes<TYPE>(u, hbm, hm, grid, bh, bl, mults, d, dmin);
+        /* block q of the scale step: with a minimum, d (even) and dmin (odd) of
+         * token group q / 2 of a pair; else d of token group q of four */
+        const float sb = kHasMin<TYPE> ? __uint_as_float((__float_as_uint(d) & ~hbm) | (__float_as_uint(dmin) & hbm)) : d;
+        if (b + 1 < B) {
+            fetch_acts(b + 1, buf ^ 1);
+            fetch_regs(b + 1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+
+        /* A slot is one matrix step of tile i and a slice of the block terms of
+         * tile i - 1 beside it (the operand reads of the next tile ride along):
+         * left to the scheduler, the products of a tile and its terms form
+         * separate runs, and both waves of a SIMD meet in the same one. */
+        constexpr int kPer = kGemmPlanes<TYPE> >= 2 ? 2 : 1;
+        constexpr int kFirst = kHasMin<TYPE> ? 1 : 0;
+        constexpr int kSlots = 4 * kPer + kFirst;
+        constexpr int kGroups = kHasMin<TYPE> ? 2 : 4; /* token groups of a scale step */
+        constexpr int kSlices = kHasMin<TYPE> ? 6 : 4;
+        i32x4 wsum[2], lsum[2], A[2][4];
+        f32x4 msum[2];
+        f32x16 da;
+        f16x8 ga[2];
+        float as[2];
+        float tf[4], tm[4];
+        auto read_a = [&](int i, int p) {
+            A[i & 1][p] = *reinterpret_cast<const i32x4 *>(&act[buf][16 * i + c16][16 * ((4 * p + 2 * hb + h) ^ c16)]);
+        };
+        auto read_rest = [&](int i) {
+            if (i % kGroups == 0)
+                as[(i / kGroups) & 1] = ascale[buf][16 * (i + (kHasMin<TYPE> ? q >> 1 : q)) + c16];
+            if constexpr (kHasMin<TYPE>)
+                ga[i & 1] = *reinterpret_cast<const f16x8 *>(&gsum[buf][16 * i + c16][8 * hb]);
+        };
+        auto slot = [&](int i, int sl) {
+            const int k = i & 1;
+            if (kFirst && sl == 0) {
+                if constexpr (kHasMin<TYPE>)
+                    msum[k] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ga[k], mults, f32x4{}, 0, 0, 0);
+                return;
+            }
+            const int p = (sl - kFirst) / kPer;
+            if ((sl - kFirst) % kPer == 0)
+                wsum[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[k][p], bh[p], p ? wsum[k] : i32x4{}, 0, 0, 0);
+            else
+                lsum[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[k][p], bl[p], p ? lsum[k] : i32x4{}, 0, 0, 0);
+        };
+        /* one operation of the reference's block term for the lane's 4 outputs
+         * of tile i (token 16 i + 4 q + e) */
+        auto slice = [&](int i, int sl) {
+            const int k = i & 1, at = 4 * (kHasMin<TYPE> ? 2 * (i & 1) : i & 3);
+            const int op = kHasMin<TYPE> ? sl : (sl < 3 ? sl : 5);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (op == 0) {
+                    int ws;
+                    if constexpr (TYPE == Q38_GGML_Q4_K) ws = wsum[k][e] * 8 + lsum[k][e];
+                    else if constexpr (TYPE == Q38_GGML_Q3_K) ws = -wsum[k][e];
+                    else if constexpr (kPer == 1) ws = wsum[k][e];
+                    else ws = wsum[k][e] * 128 + lsum[k][e];
+                    tf[e] = __int_as_float(ws);
+                } else if (op == 1) {
+                    tf[e] = (float)__float_as_int(tf[e]);
+                } else if (op == 2) {
+                    tf[e] = da[at + e] * tf[e];
+                } else if (op == 3) {
+                    tm[e] = da[at + 4 + e] * msum[k][e];
+                } else if (op == 4) {
+                    tf[e] = tf[e] - tm[e];
+                } else {
+                    total[i][e] = total[i][e] + tf[e];
+                }
+            }
+        };
+        auto scale_step = [&](int i) { /* for tiles i .. i + kGroups - 1 */
+            da = __builtin_amdgcn_mfma_f32_16x16x1f32(as[(i / kGroups) & 1], sb, f32x16{}, 0, 0, 0);
+        };
+        read_rest(0);
+#pragma unroll
+        for (int p = 0; p < 4; ++p) read_a(0, p);
+#pragma unroll
+        for (int i = 0; i < kTiles; ++i) {
+#pragma unroll
+            for (int sl = 0; sl < kSlots; ++sl) {
+                slot(i, sl);
+                if (i + 1 < kTiles) {
+                    if (sl < 4) read_a(i + 1, sl);
+                    if (sl == 3) read_rest(i + 1);
+                }
+                /* slices start after the first slot: the previous tile's last
+                 * products have then left the matrix unit */
+                if (i > 0 && sl > 0) {
+#pragma unroll
+                    for (int w = (sl - 1) * kSlices / (kSlots - 1); w < sl * kSlices / (kSlots - 1); ++w) slice(i - 1, w);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (i % kGroups == 0) scale_step(i); /* the terms of tile i - 1, which used the last one, are done */
+        }
+#pragma unroll
+        for (int w = 0; w < kSlices; ++w) slice(kTiles - 1, w);
+    }
+
+#pragma unroll
+    for (int i = 0; i < kTiles; ++i) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int tok = t0 + 16 * i + 4 * q + e;
+            if (row < rows && tok < tok_end) out[(size_t)tok * rows + row] = total[i][e];
+        }
+    }
+}
+
 /* The matrix-unit form with the blocks of a row split over the waves, for
  * grids that the 128-row x 64-token tiles would leave small (few rows or
  * few tokens): a workgroup of W waves (16, 8 or 4 as the grid has at most
@@ -1458,7 +1938,7 @@ Q38_DEV void gemm_ks_q8k(const q38_gemv_args &a) {
     const int rows = a.rows[mat];
     const int row0 = ((int)blockIdx.x - a.wg_begin[mat]) * Q38_GEMM_KS_ROWS;
     const int rowc = min(row0 + (lane & 31), rows - 1);
-    const int t0 = blockIdx.y * Q38_GEMM_KS_TOKENS;
+    const int t0 = a.tok_begin + blockIdx.y * Q38_GEMM_KS_TOKENS;
     const int T = a.n_tokens;
     const int8_t *quants = static_cast<const int8_t *>(a.q8k);
     const int16_t *sums = reinterpret_cast<const int16_t *>(quants + (size_t)T * width);
@@ -1533,7 +2013,7 @@ extern "C" __global__ __launch_bounds__(256) void q38_gemm_q8k_iq4nl(q38_gemv_ar
     const int rows = a.rows[0];
     const int row = blockIdx.x * kGemmRows + wave * 32 + (lane & 31);
     const int rowc = min(row, rows - 1);
-    const int t0 = blockIdx.y * kGemmTokens;
+    const int t0 = a.tok_begin + blockIdx.y * kGemmTokens;
     const int T = a.n_tokens;
     const int8_t *quants = static_cast<const int8_t *>(a.q8k);
     const int16_t *sums = reinterpret_cast<const int16_t *>(quants + (size_t)T * width);
@@ -1664,6 +2144,22 @@ extern "C" __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
 extern "C" __global__ __launch_bounds__(256) void q38_gemm_q8k_iq3s(q38_gemv_args a) { gemm_q8k<Q38_GGML_IQ3_S>(a); }
 extern "C" __global__ __launch_bounds__(256) void q38_gemm_q8k_iq1s(q38_gemv_args a) { gemm_q8k<Q38_GGML_IQ1_S>(a); }
 extern "C" __global__ __launch_bounds__(256) void q38_gemm_q8k_iq1m(q38_gemv_args a) { gemm_q8k<Q38_GGML_IQ1_M>(a); }
+#define Q38_GEMM_WIDE(name, T)                                                                                    \
+    extern "C" __global__ __launch_bounds__(kWideThreads, 2) void q38_gemm_wide_q8k_##name(q38_gemv_args a) {      \
+        gemm_wide_q8k<T, Q38_GEMM_WIDE_TOKENS>(a);                                                                \
+    }
+Q38_GEMM_WIDE(q4k, Q38_GGML_Q4_K)
+Q38_GEMM_WIDE(q5k, Q38_GGML_Q5_K)
+Q38_GEMM_WIDE(q6k, Q38_GGML_Q6_K)
+Q38_GEMM_WIDE(q3k, Q38_GGML_Q3_K)
+Q38_GEMM_WIDE(q2k, Q38_GGML_Q2_K)
+Q38_GEMM_WIDE(iq4xs, Q38_GGML_IQ4_XS)
+Q38_GEMM_WIDE(iq2xxs, Q38_GGML_IQ2_XXS)
+Q38_GEMM_WIDE(iq2xs, Q38_GGML_IQ2_XS)
+Q38_GEMM_WIDE(iq2s, Q38_GGML_IQ2_S)
+Q38_GEMM_WIDE(iq3xxs, Q38_GGML_IQ3_XXS)
+Q38_GEMM_WIDE(iq3s, Q38_GGML_IQ3_S)
+#undef Q38_GEMM_WIDE
 #define Q38_GEMM_KS(name, T)                                                                                      \
     extern "C" __global__ __launch_bounds__(64 * Q38_GEMM_KS_WAVES) void q38_gemm_ks_q8k_##name(q38_gemv_args a) { \
         gemm_ks_q8k<T, Q38_GEMM_KS_WAVES>(a);                                                                     \
@@ -1815,7 +2311,6 @@ extern "C" __global__ __launch_bounds__(256) void q38_gemv_f32_bf16(q38_gemv_f32
  * 256 threads; width a multiple of 64.
  */
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 template <int TYPE> struct F32wParts { static constexpr int n = 1; };
 template <> struct F32wParts<Q38_GGML_F16> { static constexpr int n = 2; };

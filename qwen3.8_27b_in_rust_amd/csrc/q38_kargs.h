@@ -337,6 +337,10 @@ typedef struct {
 #define Q38_GEMM_IQ4NL_MIN_TOKENS 32
 #define Q38_GEMM_ROWS 128
 #define Q38_GEMM_TOKENS 64
+/* Long prompts: 128 x 256 tiles (q38_gemm_wide_q8k_*: grid (8 ceil(tiles /
+ * 8)), 512 threads, up to Q38_GEMV_MAX_MATS matrices, matrix m on 128-row
+ * tiles wg_begin[m] .. wg_begin[m+1]-1). */
+#define Q38_GEMM_WIDE_TOKENS 256
 /* Where that grid holds few workgroups (few rows or tokens), the blocks of a
  * row are split over the waves instead (q38_gemm_ks_q8k_*: grid (ceil(rows /
  * 32), ceil(T / 32)), Q38_GEMM_KS_WAVES waves of 64 threads, the same
@@ -365,6 +369,10 @@ typedef struct {
     int32_t n_tokens;
     int32_t tok_pass;
     int32_t tok_groups;
+    /* the matrix-unit forms: the launch's tokens tok_begin .. tok_end-1 of
+     * the n_tokens (tok_begin a multiple of Q38_GEMM_WIDE_TOKENS) */
+    int32_t tok_begin;
+    int32_t tok_end;
 } q38_gemv_args;
 
 /* f32-input projections (F32, F16, BF16, Q8_0 weights): the GEMV, grid

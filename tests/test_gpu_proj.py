@@ -284,6 +284,40 @@ def test_multi_matrices_share_the_split_block_launch(ctx, ref, name):
             assert np.array_equal(got.view(np.uint32), single.download().view(np.uint32)), r
 
 
+@pytest.mark.parametrize("name,rows,T,kern", [
+    ("Q4_K", [16384], 513, "wide"),           # two full token tiles, one token left to the split-block form
+    ("Q6_K", [16384 - 127], 500, "wide"),     # a ragged row tile, a ragged token tile, no rest
+    ("Q5_K", [12288, 1024, 4096], 511, "wide"),  # three matrices in a launch
+    ("Q2_K", [16384], 768, "wide"), ("Q3_K", [16300], 520, "wide"), ("IQ4_XS", [16384], 400, "wide"),
+    ("IQ2_S", [16384], 512, "wide"), ("IQ3_S", [16384], 640, "wide"), ("IQ2_XXS", [16384], 512, "wide"),
+    ("IQ2_XS", [16384], 512, "wide"), ("IQ3_XXS", [16384], 512, "wide"),
+    ("IQ1_S", [16384], 512, ""), ("Q4_K", [16384], 129, ""),  # no such form; too few tokens
+])
+def test_wide_tiles_bit_exact(ctx, ref, name, rows, T, kern):
+    """The 128 x 256 tiles with the rest of the tokens on the other forms:
+    every output is the oracle's bit for bit.  Scales down to f16 subnormals
+    (random blocks) and one token of zeros among the inputs."""
+    ty = TYPES[name]
+    W = 768
+    x = _activations(T, W, 0x51333C00 + T)
+    x[T // 2] = 0
+    d_q = _quantize_on_device(ctx, x)
+    q8 = ref.quantize_q8_k(x)
+    wbs = [_random_kquant(ty, r, W, 0x51333C01 + ty + r) for r in rows]
+    d_ws = [ctx.array(wb, np.uint8) for wb in wbs]
+    d_os = [ctx.empty((T, r)) for r in rows]
+    call = lambda: ctx.gemv_q8_k_multi(ty, rows, W, d_ws, d_q, T, d_os)
+    if kern:
+        assert _ran(ctx, "q38_gemm_wide_q8k_" + name.lower().replace("_", ""), call)
+    else:
+        call()
+    for wb, r, d_o in zip(wbs, rows, d_os):
+        want = ref.gemv_q8_k(ty, wb, q8, T, W, threads=16)
+        assert np.array_equal(d_o.download().view(np.uint32), want.view(np.uint32)), r
+    for arr in [d_q, *d_ws, *d_os]:
+        arr.free()
+
+
 F32_PATH_SHAPES = [(48, HIDDEN, 1), (48, HIDDEN, 3), (257, 1024, 9), (5, 6144, 17), (1031, 2048, 1),
                    (48, HIDDEN, 64), (300, 1024, 100), (129, 768, 33), (64, 320, 16), (40, 1032, 20), (37, 64, 5),
                    (19, 17408, 2), (70, 14528, 3), (33, 6144, 15), (2048, 256, 512), (100, 1024, 9),
