@@ -97,15 +97,23 @@ Q38_DEV void decode_rows(DecodeState &st, const f32x4 (&q0)[Q38_ATTN_GROUP],
     }
 }
 
-/* RoPE angles of one position, once: pair p gets theta_p = position *
- * scale^p by p repeated f32 multiplications (the reference's rounding), and
- * cs[p] = (cos, sin) of it; lane p < 32 of the calling wave forms pair p. */
+/* RoPE angles of one position: pair p gets theta_p = position * scale^p by p
+ * repeated f32 multiplications (the reference's rounding), and cs[p] = (cos,
+ * sin) of it; lane p < 32 of the calling half-wave forms pair p, every lane
+ * running the whole chain and keeping its own term of it (a loop of p steps
+ * costs a branch a step). */
 Q38_DEV void q38_rope_table(float (*cs)[2], int lane, int position, float theta_scale) {
+    float theta = (float)position, mine = theta;
+#pragma unroll
+    for (int i = 1; i < 32; ++i) {
+        theta *= theta_scale;
+        mine = lane == i ? theta : mine;
+    }
+    float sine, cosine;
+    sincosf(mine, &sine, &cosine);
     if (lane < 32) {
-        float theta = (float)position;
-        for (int i = 0; i < lane; ++i) theta *= theta_scale;
-        cs[lane][0] = cosf(theta);
-        cs[lane][1] = sinf(theta);
+        cs[lane][0] = cosine;
+        cs[lane][1] = sine;
     }
 }
 
@@ -146,9 +154,7 @@ Q38_DEV void q38_norm_rope8(f32x4 &x0, f32x4 &x1, f32x4 w0, f32x4 w1, int li, co
     double ss = 0.0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) ss += (double)x0[c] * (double)x0[c] + (double)x1[c] * (double)x1[c];
-#pragma unroll
-    for (int m = 16; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
-    const float scale = q38_rms_scale_of(ss);
+    const float scale = q38_rms_scale_of(q38_sum32_f64(ss));
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
         x0[c] = x0[c] * scale * w0[c];
@@ -226,6 +232,38 @@ Q38_DEV void decode_split(const q38_decode_args &a) {
      * (each head's q followed by its gate) */
     const int q_stride = kPre ? 2 * Q38_ATTN_HEAD_DIM : Q38_ATTN_HEAD_DIM;
     const float *qb = a.q + ((size_t)b * Q38_ATTN_HEADS + j * Q38_ATTN_GROUP) * q_stride;
+    auto load_q = [&]() {
+#pragma unroll
+        for (int hh = 0; hh < Q38_ATTN_GROUP; ++hh) {
+            q0[hh] = q38_ld4(qb + hh * q_stride + d0);
+            q1[hh] = q38_ld4(qb + hh * q_stride + d1);
+        }
+    };
+    /* With the pre step fused (RMSNorm and RoPE, ops.rs:832-856), half-wave hw
+     * < 6 forms query head hw and half-wave 6, in the split holding `pos`, the
+     * new key row, both into LDS; every half-wave forms the RoPE table for
+     * itself, so one barrier serves them and the page ids.  (Each half-wave
+     * forming all six heads, behind a barrier for one shared table, took 3.8 us
+     * more: full_core of one token 16.8 against 13.0 us at 1K, 51.5 against
+     * 48.1 at 32K.)  The row loads come first: their inputs, like the rows
+     * below, are in flight while the table is formed. */
+    __shared__ __attribute__((aligned(16))) float k_formed[Q38_ATTN_HEAD_DIM];
+    __shared__ __attribute__((aligned(16))) float q_formed[kPre ? Q38_ATTN_GROUP : 1][Q38_ATTN_HEAD_DIM];
+    __shared__ float rope_cs[kPre ? 2 * NW : 1][32][2];
+    static_assert(2 * NW > Q38_ATTN_GROUP, "a half-wave per query head and one for the key");
+    const int hw = tid >> 5;
+    const bool holds_pos = pos >= t_begin && pos < t_end;
+    const bool forms_key = kPre && hw == Q38_ATTN_GROUP && a.k_new != nullptr && holds_pos;
+    const bool forms = kPre && (hw < Q38_ATTN_GROUP || forms_key);
+    f32x4 px0 = {0.f, 0.f, 0.f, 0.f}, px1 = px0, pw0 = px0, pw1 = px0;
+    if (forms) {
+        const float *src = forms_key ? a.k_new + (size_t)b * Q38_ATTN_KV_DIM + j * Q38_ATTN_HEAD_DIM : qb + hw * q_stride;
+        const float *w = forms_key ? a.k_norm : a.q_norm;
+        px0 = q38_ld4(src + d0);
+        px1 = q38_ld4(src + d1);
+        pw0 = q38_ld4(w + d0);
+        pw1 = q38_ld4(w + d1);
+    }
     if (kArgPages) {
         /* software pipeline start: wave w's half-page w lies in the split's
          * page 0 or 1, whose ids come with the launch, so these loads issue at
@@ -240,33 +278,21 @@ Q38_DEV void decode_split(const q38_decode_args &a) {
                                 Q38_ATTN_HEAD_DIM + (size_t)(hp0 & 1) * 8 * Q38_ATTN_HEAD_DIM;
         load_rows(K, a.kpool, base, lane_off);
         load_rows(V, a.vpool, base, lane_off);
-#pragma unroll
-        for (int hh = 0; hh < Q38_ATTN_GROUP; ++hh) {
-            q0[hh] = q38_ld4(qb + hh * q_stride + d0);
-            q1[hh] = q38_ld4(qb + hh * q_stride + d1);
-        }
+        if (!kPre) load_q();
         pages[tid] = my_page;
     } else {
-#pragma unroll
-        for (int hh = 0; hh < Q38_ATTN_GROUP; ++hh) {
-            q0[hh] = q38_ld4(qb + hh * q_stride + d0);
-            q1[hh] = q38_ld4(qb + hh * q_stride + d1);
-        }
+        if (!kPre) load_q();
         if (tid < n_split_pages) pages[tid] = pt[(t_begin >> 4) + tid];
     }
-    /* with the pre step fused, the split holding `pos` forms the new key row
-     * (RMSNorm and RoPE of the raw key, ops.rs:844-856) in LDS; it is
-     * appended below and scored from there */
-    __shared__ __attribute__((aligned(16))) float k_formed[Q38_ATTN_HEAD_DIM];
-    __shared__ float rope_cs[32][2];
-    const bool holds_pos = pos >= t_begin && pos < t_end;
     if (kPre) {
-        if (wave == NW - 1) q38_rope_table(rope_cs, lane, pos, a.theta_scale);
-        __syncthreads();
-        if (a.k_new != nullptr && holds_pos && wave == 0) {
-            f32x4 x = q38_ld4(a.k_new + (size_t)b * Q38_ATTN_KV_DIM + j * Q38_ATTN_HEAD_DIM + 4 * lane);
-            q38_norm_rope4_cs(x, q38_ld4(a.k_norm + 4 * lane), lane, rope_cs);
-            q38_st4(&k_formed[4 * lane], x);
+        q38_rope_table(rope_cs[hw], li, pos, a.theta_scale);
+        __builtin_amdgcn_wave_barrier(); /* the lanes of a half-wave read each other's entries below */
+        if (forms) {
+            q38_norm_rope8(px0, px1, pw0, pw1, li, rope_cs[hw]);
+            const float unit = forms_key ? 1.0f : Q38_SCORE_LOG2;
+            float *dst = forms_key ? k_formed : q_formed[hw];
+            q38_st4(dst + d0, px0 * unit);
+            q38_st4(dst + d1, px1 * unit);
         }
     }
     __syncthreads();
@@ -296,20 +322,12 @@ Q38_DEV void decode_split(const q38_decode_args &a) {
         load_rows(V, a.vpool, base, lane_off);
     }
 
-    if (kPre) {
-        /* the group's query heads RMSNormed and rotated here (ops.rs:832-856;
-         * the same arithmetic as q38_attn_pre), each half-wave holding a whole
-         * head */
-        const f32x4 w0 = q38_ld4(a.q_norm + d0), w1 = q38_ld4(a.q_norm + d1);
 #pragma unroll
-        for (int hh = 0; hh < Q38_ATTN_GROUP; ++hh) {
-            q38_norm_rope8(q0[hh], q1[hh], w0, w1, li, rope_cs);
-            q0[hh] *= Q38_SCORE_LOG2;
-            q1[hh] *= Q38_SCORE_LOG2;
-        }
-    } else {
-#pragma unroll
-        for (int hh = 0; hh < Q38_ATTN_GROUP; ++hh) {
+    for (int hh = 0; hh < Q38_ATTN_GROUP; ++hh) {
+        if (kPre) {
+            q0[hh] = q38_ld4(&q_formed[hh][d0]);
+            q1[hh] = q38_ld4(&q_formed[hh][d1]);
+        } else {
             q0[hh] *= Q38_SCORE_LOG2;
             q1[hh] *= Q38_SCORE_LOG2;
         }

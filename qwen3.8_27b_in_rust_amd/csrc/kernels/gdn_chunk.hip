@@ -680,8 +680,7 @@ extern "C" __global__ __launch_bounds__(256) void q38_gdn_post(q38_gdn_post_args
     for (int p = 0; p < 2; ++p) {
         double ss = (double)x[p].x * (double)x[p].x + (double)x[p].y * (double)x[p].y +
                     (double)x[p].z * (double)x[p].z + (double)x[p].w * (double)x[p].w;
-#pragma unroll
-        for (int m = 16; m >= 1; m >>= 1) ss += __shfl_xor(ss, m, 64);
+        ss = q38_sum32_f64(ss);
         const float mean = (float)(ss / (double)D);
         const float scale = 1.0f / sqrtf(mean + 1e-6f);
         f32x4 y;

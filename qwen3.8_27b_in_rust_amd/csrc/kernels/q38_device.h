@@ -100,11 +100,41 @@ Q38_DEV f32x4 q38_fma4(float s, f32x4 v, f32x4 acc) {
     return acc;
 }
 
-/* f64 all-reduce over the wave (64 lanes) through ds_swizzle-free shuffles. */
-Q38_DEV double q38_wave_sum_f64(double x) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) x += __shfl_xor(x, m, 64);
+/* f64 all-reduce (sum) over each row of 16 lanes, each half-wave and the wave
+ * with the DPP and permlane moves of the f32 forms above, a word at a time.
+ * A sum by __shfl_xor of doubles is two LDS permutes per step, and the decode
+ * kernels run several of them in a row before their first row is scored:
+ * moved to registers, with the query heads shared out among the half-waves
+ * (decode_split), a one-token full_core at 1K takes 13.0 us against 16.8. */
+template <int CTRL>
+Q38_DEV double q38_dpp_f64(double x) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xF, 0xF, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+}
+Q38_DEV double q38_sum16_f64(double x) {
+    x += q38_dpp_f64<0xB1>(x);
+    x += q38_dpp_f64<0x4E>(x);
+    x += q38_dpp_f64<0x141>(x);
+    x += q38_dpp_f64<0x140>(x);
     return x;
+}
+Q38_DEV double q38_sum32_f64(double x) {
+    x = q38_sum16_f64(x);
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)b, (uint32_t)b, false, false);
+    auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    return __builtin_bit_cast(double, (uint64_t)hi[0] << 32 | lo[0]) +
+           __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]);
+}
+Q38_DEV double q38_wave_sum_f64(double x) {
+    x = q38_sum32_f64(x);
+    const uint64_t b = __builtin_bit_cast(uint64_t, x);
+    auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)b, (uint32_t)b, false, false);
+    auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)(b >> 32), (uint32_t)(b >> 32), false, false);
+    return __builtin_bit_cast(double, (uint64_t)hi[0] << 32 | lo[0]) +
+           __builtin_bit_cast(double, (uint64_t)hi[1] << 32 | lo[1]);
 }
 
 /* s_waitcnt immediate (gfx9 encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4,
