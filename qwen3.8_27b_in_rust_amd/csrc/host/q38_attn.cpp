@@ -2281,8 +2281,25 @@ int q38_gemv_f32(q38_ctx *ctx, int ggml_type, int rows, int width, const void *d
         s.rows = rows;
         s.width = width;
         s.n_tokens = n_tokens;
-        return ctx->launch(ctx->f_gemm_f32s[ti], (unsigned)((rows + 63) / 64), (unsigned)((n_tokens + 31) / 32), 1,
-                           256, &s);
+        /* Few rows (the 48-row beta / alpha projections) are too few tiles for
+         * the matrix unit to beat the GEMV's row per wave, whose loads are
+         * contiguous, while that grid is at most two workgroups per CU: 48 x
+         * 5120 F32 at 4 / 32 / 331 tokens 9.3 / 15.3 / 27.9 us against 28 / 40 /
+         * 40 (78.7 against 41.5 at 1024), BF16 9.9 / 15.9 / 28.6 against 18 / 30 /
+         * 30; 1024 x 5120 F32 at 16 tokens 16.9 against 33 (BF16 at 32: 32.9
+         * against 30.4) */
+        if (ti < 3 && row_groups * tok_groups <= 2L * ctx->cu_count) {
+            s.form = Q38_F32S_ROWS;
+            return ctx->launch(ctx->f_gemm_f32s[ti], (unsigned)row_groups, (unsigned)tok_groups, 1, 256, &s);
+        }
+        /* 64 rows a workgroup, or, where that leaves half the CUs without one,
+         * 32 rows on twice the waves */
+        const long toks = ((long)n_tokens + 31) / 32;
+        const bool few = 2 * (((long)rows + 63) / 64 * toks) <= (long)ctx->cu_count;
+        const int tile_rows = few ? 32 : 64;
+        s.form = few ? Q38_F32S_8_WAVES : Q38_F32S_4_WAVES;
+        return ctx->launch(ctx->f_gemm_f32s[ti], (unsigned)((rows + tile_rows - 1) / tile_rows), (unsigned)toks, 1,
+                           few ? 512 : 256, &s);
     }
     q38_gemv_f32_args a;
     memset(&a, 0, sizeof(a));

@@ -2647,100 +2647,125 @@ Q38_DEV void f32s_parts(const F32sRaw<TYPE> &r, int sb, const uint8_t *p, u32x4 
     }
 }
 
-template <int TYPE>
-Q38_DEV void gemm_f32s(const q38_gemv_f32_args &a) {
+/* RT row tiles of 32 per workgroup, k split over W waves, DEPTH 32-wide slices
+ * of k in flight per wave.  Two instances: (2, 4, 1), and where that grid
+ * leaves half the CUs idle or more (1, 8, 4).  Bound by the CU's load path: a
+ * lane's 16-byte pieces lie a row apart, and few rows are few CUs -- 48 x 5120
+ * F32 at 32 tokens, one workgroup, 50 us; on the second form 40. */
+template <int TYPE, int RT, int W, int DEPTH>
+Q38_DEV void gemm_f32s_tile(const q38_gemv_f32_args &a, float *red) {
     constexpr int PW = F32wParts<TYPE>::n;
-    __shared__ float red[3][2][16][64]; /* waves 1-3: [wave - 1][tile][element][lane] */
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
     const int h = lane >> 5, l32 = lane & 31;
-    const int rows = a.rows, W = a.width, T = a.n_tokens;
-    const int row0 = blockIdx.x * 64;
+    const int rows = a.rows, T = a.n_tokens;
+    const int row0 = blockIdx.x * 32 * RT;
     const int t0 = blockIdx.y * 32;
-    const int n_slices = W / 32;
-    const int s_begin = n_slices * wave / 4, s_end = n_slices * (wave + 1) / 4;
-    const float *xp = a.x + (size_t)min(t0 + l32, T - 1) * W + 16 * h;
-    const uint8_t *wp[2];
+    const int n_slices = a.width / 32;
+    const int s_begin = n_slices * wave / W, s_end = n_slices * (wave + 1) / W;
+    const float *xp = a.x + (size_t)min(t0 + l32, T - 1) * a.width + 16 * h;
+    const uint8_t *wp[RT];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) wp[r] = a.weights + (size_t)min(row0 + 32 * r + l32, rows - 1) * a.row_bytes;
+    for (int r = 0; r < RT; ++r) wp[r] = a.weights + (size_t)min(row0 + 32 * r + l32, rows - 1) * a.row_bytes;
 
-    f32x4 xc[4], xn[4];
-    F32sRaw<TYPE> wc[2], wn[2];
-    auto load = [&](int sl, f32x4(&xr)[4], F32sRaw<TYPE>(&wr)[2]) {
+    /* the slice being computed and the DEPTH after it */
+    f32x4 xs[DEPTH + 1][4];
+    F32sRaw<TYPE> ws[DEPTH + 1][RT];
+    auto load = [&](int sl, int at) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) xr[i] = q38_ld4(xp + (size_t)sl * 32 + 4 * i);
+        for (int i = 0; i < 4; ++i) xs[at][i] = q38_ld4(xp + (size_t)sl * 32 + 4 * i);
 #pragma unroll
-        for (int r = 0; r < 2; ++r) f32s_load<TYPE>(wp[r], sl, h, wr[r]);
+        for (int r = 0; r < RT; ++r) f32s_load<TYPE>(wp[r], sl, h, ws[at][r]);
     };
-    f32x16 acc[2];
+    f32x16 acc[RT];
 #pragma unroll
-    for (int r = 0; r < 2; ++r)
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[r][e] = 0.0f;
-    if (s_begin < s_end) load(s_begin, xc, wc);
-    for (int sl = s_begin; sl < s_end; ++sl) {
-        if (sl + 1 < s_end) load(sl + 1, xn, wn);
-        f32x16 blk[2];
-        if constexpr (TYPE == Q38_GGML_Q8_0) {
 #pragma unroll
-            for (int r = 0; r < 2; ++r)
+    for (int k = 0; k < DEPTH; ++k)
+        if (s_begin + k < s_end) load(s_begin + k, k);
+    for (int s0 = s_begin; s0 < s_end; s0 += DEPTH + 1) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e) blk[r][e] = 0.0f;
-        }
+        for (int k = 0; k <= DEPTH; ++k) {
+            const int sl = s0 + k;
+            if (sl >= s_end) break;
+            if (sl + DEPTH < s_end) load(sl + DEPTH, (k + DEPTH) % (DEPTH + 1));
+            f32x16 blk[RT];
+            if constexpr (TYPE == Q38_GGML_Q8_0) {
 #pragma unroll
-        for (int sb = 0; sb < 2; ++sb) {
-            float v[8];
+                for (int r = 0; r < RT; ++r)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = xc[2 * sb + (i >> 2)][i & 3];
-            u32x4 ax[3];
-            split_parts<3>(v, ax);
+                    for (int e = 0; e < 16; ++e) blk[r][e] = 0.0f;
+            }
 #pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                u32x4 bw[PW];
-                f32s_parts<TYPE>(wc[r], sb, wp[r] + (size_t)sl * 34 + 2 + 16 * h, bw);
-                if constexpr (TYPE == Q38_GGML_Q8_0) blk[r] = f32w_products<PW>(ax, bw, blk[r]);
-                else acc[r] = f32w_products<PW>(ax, bw, acc[r]);
+            for (int sb = 0; sb < 2; ++sb) {
+                float v[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = xs[k][2 * sb + (i >> 2)][i & 3];
+                u32x4 ax[3];
+                split_parts<3>(v, ax);
+#pragma unroll
+                for (int r = 0; r < RT; ++r) {
+                    u32x4 bw[PW];
+                    f32s_parts<TYPE>(ws[k][r], sb, wp[r] + (size_t)sl * 34 + 2 + 16 * h, bw);
+                    if constexpr (TYPE == Q38_GGML_Q8_0) blk[r] = f32w_products<PW>(ax, bw, blk[r]);
+                    else acc[r] = f32w_products<PW>(ax, bw, acc[r]);
+                }
+            }
+            if constexpr (TYPE == Q38_GGML_Q8_0) {
+#pragma unroll
+                for (int r = 0; r < RT; ++r) {
+                    /* this lane's output column is its own row l % 32 of tile r */
+                    const float d = q38_f16(ws[k][r].d);
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[r][e] = __builtin_fmaf(d, blk[r][e], acc[r][e]);
+                }
             }
         }
-        if constexpr (TYPE == Q38_GGML_Q8_0) {
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                /* this lane's output column is its own row l % 32 of tile r */
-                const float d = q38_f16(wc[r].d);
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[r][e] = __builtin_fmaf(d, blk[r][e], acc[r][e]);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) xc[i] = xn[i];
-#pragma unroll
-        for (int r = 0; r < 2; ++r) wc[r] = wn[r];
     }
+    /* waves 1 .. W-1: [wave - 1][tile][element][lane] */
+    auto at = [&](int w, int r, int e) { return ((w * RT + r) * 16 + e) * 64 + lane; };
     if (wave > 0) {
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
+        for (int r = 0; r < RT; ++r)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) red[wave - 1][r][e][lane] = acc[r][e];
+            for (int e = 0; e < 16; ++e) red[at(wave - 1, r, e)] = acc[r][e];
     }
     __syncthreads();
     if (wave != 0) return;
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
+    for (int r = 0; r < RT; ++r) {
         const int row = row0 + 32 * r + l32;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
-            const float v = ((acc[r][e] + red[0][r][e][lane]) + red[1][r][e][lane]) + red[2][r][e][lane];
+            float v = acc[r][e];
+#pragma unroll
+            for (int w = 0; w < W - 1; ++w) v += red[at(w, r, e)];
             const int tok = t0 + 8 * (e >> 2) + 4 * h + (e & 3);
             if (row < rows && tok < T) a.out[(size_t)tok * rows + row] = v;
         }
     }
 }
 
-extern "C" __global__ __launch_bounds__(256) void q38_gemm_f32s_f32(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_F32>(a); }
-extern "C" __global__ __launch_bounds__(256) void q38_gemm_f32s_f16(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_F16>(a); }
-extern "C" __global__ __launch_bounds__(256) void q38_gemm_f32s_bf16(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_BF16>(a); }
-extern "C" __global__ __launch_bounds__(256) void q38_gemm_f32s_q8_0(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_Q8_0>(a); }
+template <int TYPE>
+Q38_DEV void gemm_f32s(const q38_gemv_f32_args &a) {
+    __shared__ float red[7 * 16 * 64];
+    static_assert(3 * 2 <= 7, "either form's partial sums");
+    if (a.form == Q38_F32S_8_WAVES) {
+        gemm_f32s_tile<TYPE, 1, 8, 4>(a, red);
+    } else if (a.form == Q38_F32S_ROWS) {
+        if constexpr (TYPE != Q38_GGML_Q8_0) gemv_f32<TYPE>(a); /* Q8_0 has no such launch */
+    } else {
+        gemm_f32s_tile<TYPE, 2, 4, 1>(a, red);
+    }
+}
+
+extern "C" __global__ __launch_bounds__(512) void q38_gemm_f32s_f32(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_F32>(a); }
+extern "C" __global__ __launch_bounds__(512) void q38_gemm_f32s_f16(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_F16>(a); }
+extern "C" __global__ __launch_bounds__(512) void q38_gemm_f32s_bf16(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_BF16>(a); }
+extern "C" __global__ __launch_bounds__(512) void q38_gemm_f32s_q8_0(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_Q8_0>(a); }
 
 /*
  * Q8_0 weights below 16 tokens: a workgroup of 4 waves takes 4 RW rows (RW
