@@ -1795,7 +1795,13 @@ static int gdn_chunked(q38_ctx *ctx, int n_seq, int n_tokens, float *d_state, in
     for (int c0 = 0; c0 < n_chunks; c0 += Q38_GDN_STAGE_CHUNKS) {
         a.chunk0 = c0;
         a.n_chunks = std::min(Q38_GDN_STAGE_CHUNKS, n_chunks - c0);
-        if (ctx->launch(ctx->f_chunk_prep, Q38_LIN_QK_HEADS, a.n_chunks, n_seq, 512, &a)) return -1;
+        /* one workgroup fits a CU: split the 3 value heads of each while every
+         * part still starts at once (5 chunks of one sequence in thirds, 8 in
+         * two): linear_core of 16 / 100 / 331 tokens 34.9 / 42.9 / 73.6 us
+         * against 55.1 / 63.4 / 83.4 undivided */
+        const long base = (long)Q38_LIN_QK_HEADS * a.n_chunks * n_seq;
+        a.prep_parts = 3 * base <= (long)ctx->cu_count ? 3 : 2 * base <= (long)ctx->cu_count ? 2 : 1;
+        if (ctx->launch(ctx->f_chunk_prep, Q38_LIN_QK_HEADS * a.prep_parts, a.n_chunks, n_seq, 512, &a)) return -1;
         if (ctx->launch(ctx->f_chunk_scan, Q38_LIN_V_HEADS * 4, n_seq, 1, 64 * Q38_GDN_SCAN_WAVES, &a)) return -1;
     }
     return 0;
@@ -1907,9 +1913,6 @@ int q38_linear_core(q38_ctx *ctx, int n_seq, int n_tokens, const q38_linear_weig
     p.n_tokens = n_tokens;
     p.n_seq = n_seq;
     if (ctx->launch(ctx->f_gdn_pre, Q38_LIN_QKV_DIM / 1024 + 1, pre_runs, n_seq, 256, &p)) return -1;
-    if (pre_runs > 1)
-        Q38_HIP(hipMemcpyAsync(d_conv_state, conv_out, conv_floats * sizeof(float),
-                               hipMemcpyDeviceToDevice, ctx->stream));
     /* prompt: chunked recurrence, then the gated RMSNorm */
     if (gdn_chunked(ctx, n_seq, n_tokens, d_delta_state, Q38_LIN_STATE_FLOATS, x, x + Q38_LIN_QK_DIM,
                     x + 2 * Q38_LIN_QK_DIM, beta, g, o_raw, Q38_LIN_QKV_DIM, Q38_LIN_QKV_DIM, chunk_work))
@@ -1920,6 +1923,11 @@ int q38_linear_core(q38_ctx *ctx, int n_seq, int n_tokens, const q38_linear_weig
     pa.z = d_z;
     pa.norm_w = w->d_norm;
     pa.out = d_out;
+    if (pre_runs > 1) { /* the pre kernel's first run reads the state its last one writes */
+        pa.conv_src = conv_out;
+        pa.conv_dst = d_conv_state;
+        pa.conv_floats = (int64_t)conv_floats;
+    }
     /* 16 (token, value head) rows per workgroup; toks * 48 rows */
     return ctx->launch(ctx->f_gdn_post, (unsigned)(toks * (Q38_LIN_V_HEADS / 16)), 1, 1, 256, &pa);
 }

@@ -219,7 +219,10 @@ Q38_DEV void invert_unit_lower(const float (*sA)[BR], float (*sT)[C + 4], int wa
  * One workgroup per (q/k head, chunk): the 3 value heads that read q/k head
  * kh (value heads kh, kh + 16, kh + 32; ops.rs:691) share K, Q, their bf16
  * splits and the products K K^T and Q K^T; the decays, betas, T, W, U' and
- * the images are per value head, formed one head after another.
+ * the images are per value head, formed one head after another.  A head is a
+ * chain of short phases (12 us of a 42 us workgroup), so while the grid leaves
+ * CUs idle two or three workgroups share the heads and repeat the products
+ * (prep_parts).
  */
 extern "C" __global__ __launch_bounds__(kPrepThreads) void q38_gdn_chunk_prep(q38_gdn_chunk_args a) {
     constexpr int kGroup = Q38_LIN_V_HEADS / Q38_LIN_QK_HEADS;
@@ -246,7 +249,10 @@ extern "C" __global__ __launch_bounds__(kPrepThreads) void q38_gdn_chunk_prep(q3
     __bf16 *const sQh = &sVh[0][0]; /* [C][WR] */
     __bf16 *const sQl = &sVl[0][0];
 
-    const int kh = blockIdx.x;
+    /* grid x: q/k head, then part: value heads j0 .. j1-1 of the head's 3 */
+    const int kh = blockIdx.x % Q38_LIN_QK_HEADS;
+    const int per_part = (kGroup + a.prep_parts - 1) / a.prep_parts;
+    const int j0 = (int)(blockIdx.x / Q38_LIN_QK_HEADS) * per_part, j1 = min(j0 + per_part, kGroup);
     const int n = blockIdx.y;
     const int s = blockIdx.z;
     const int tid = threadIdx.x;
@@ -281,7 +287,7 @@ extern "C" __global__ __launch_bounds__(kPrepThreads) void q38_gdn_chunk_prep(q3
         kv[p] = q38_ld4(a.k + tok * a.q_stride + kh * D + 4 * col_c4());
         qv[p] = q38_ld4(a.q + tok * a.q_stride + kh * D + 4 * col_c4());
     }
-    load_v(kh);
+    load_v(kh + Q38_LIN_QK_HEADS * j0);
     /* log-decays and betas of the three heads, one token per lane; every
      * wave forms the inclusive prefix sums G of the log-decays for its own
      * use */
@@ -320,6 +326,7 @@ extern "C" __global__ __launch_bounds__(kPrepThreads) void q38_gdn_chunk_prep(q3
         split4_store(sQh + t * WR + 4 * c4, sQl + t * WR + 4 * c4, qx);
 #pragma unroll
         for (int j = 0; j < kGroup; ++j) {
+            if (j < j0 || j >= j1) continue;
             const Record rec = record_of(a, s, kh + Q38_LIN_QK_HEADS * j, n);
             const float gam = expf(__shfl(acc_g[j], t, 64));
             split4_store(rec.q_hi + t * WR + 4 * c4, rec.q_lo + t * WR + 4 * c4, gam * qx);
@@ -344,6 +351,7 @@ extern "C" __global__ __launch_bounds__(kPrepThreads) void q38_gdn_chunk_prep(q3
 
 #pragma unroll
     for (int j = 0; j < kGroup; ++j) {
+        if (j < j0 || j >= j1) continue;
         const int vh = kh + Q38_LIN_QK_HEADS * j;
         const Record rec = record_of(a, s, vh, n);
 
@@ -371,7 +379,7 @@ extern "C" __global__ __launch_bounds__(kPrepThreads) void q38_gdn_chunk_prep(q3
                 sVl[4 * c4 + e][t] = (__bf16)(vx[e] - (float)h);
             }
         }
-        if (j + 1 < kGroup) load_v(vh + Q38_LIN_QK_HEADS);
+        if (j + 1 < j1) load_v(vh + Q38_LIN_QK_HEADS);
         lds_barrier();
 
         /* A (strictly lower) into LDS and Bm (lower, with the diagonal; zero
@@ -468,7 +476,7 @@ extern "C" __global__ __launch_bounds__(kPrepThreads) void q38_gdn_chunk_prep(q3
                 for (int i = 0; i < 4; ++i) rec.u[(16 * ti + 4 * g4 + i) * D + 16 * tn + r] = acc[i];
             }
         }
-        if (j + 1 < kGroup) lds_barrier(); /* the next head reuses every per-head array */
+        if (j + 1 < j1) lds_barrier(); /* the next head reuses every per-head array */
     }
 }
 
@@ -663,11 +671,14 @@ extern "C" __global__ __launch_bounds__(64 * kScanWaves) void q38_gdn_chunk_scan
  * 128 outputs with the f64 sum of squares, weight, times silu(z).  grid
  * (n_rows / 16), 256 threads: each wave takes 4 rows, a half-wave one row
  * at a time with 4 consecutive columns per lane, both rows' loads issued
- * before the first reduction. */
+ * before the first reduction.  The launch also moves the conv state (as a copy
+ * of its own between the pre and the prep kernel it cost 1-2 us a prompt). */
 extern "C" __global__ __launch_bounds__(256) void q38_gdn_post(q38_gdn_post_args a) {
     const int lane = threadIdx.x & 63;
     const int col = 4 * (lane & 31);
     const size_t row0 = ((size_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 4 + (lane >> 5);
+    for (size_t i = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x); i < (size_t)a.conv_floats; i += 1024 * (size_t)gridDim.x)
+        q38_st4(a.conv_dst + i, q38_ld4(a.conv_src + i));
     const f32x4 nw = q38_ld4(a.norm_w + col);
     f32x4 x[2], z[2];
 #pragma unroll

@@ -169,7 +169,7 @@ typedef struct {
     int32_t n_tokens;
     int32_t n_chunks;  /* chunks of this launch: chunk0 .. chunk0 + n_chunks - 1 */
     int32_t chunk0;
-    int32_t pad_;
+    int32_t prep_parts; /* workgroups that share the 3 value heads of a (q/k head, chunk): 1-3 */
 } q38_gdn_chunk_args;
 /* chunks per prep/scan launch pair: a stage's records (16 x 48 x 158 KB, ~121 MB
  * per sequence) stay in the last-level cache between the two launches */
@@ -183,6 +183,11 @@ typedef struct {
     const float *z;    /* same layout */
     const float *norm_w; /* [128] */
     float *out;
+    /* the prompt's last conv state, from where q38_gdn_pre left it to its
+     * place (16-byte aligned; conv_floats a multiple of 4, 0: none) */
+    const float *conv_src;
+    float *conv_dst;
+    int64_t conv_floats;
 } q38_gdn_post_args;
 
 /* conv1d(k=4) with state shift, SiLU, per-head L2 norm of q and k, and the
