@@ -1753,30 +1753,44 @@ Q38_DEV void gemm_wide_q8k(const q38_gemv_args &a) {
      * tid / 2) */
     const size_t sc_at = (size_t)min(t0 + (tid & (NT - 1)), T - 1) * B;
     const size_t gs_at = (size_t)min(t0 + (tid >> 1) % NT, T - 1) * B;
-    float my_scale;
-    u32x4 my_sums = {};
+    float sc4[4];
+    u32x4 sums4[4];
     Part<TYPE> u;
-    auto fetch_regs = [&](int b) {
-        load_part<TYPE>(weights, unit0 + b, hb, h, u);
-        my_scale = scales[sc_at + b];
-        if constexpr (kHasMin<TYPE>)
-            my_sums = *reinterpret_cast<const u32x4 *>(sums + (gs_at + b) * 16 + 8 * (tid & 1));
+    auto fetch_weights = [&](int b) { load_part<TYPE>(weights, unit0 + b, hb, h, u); };
+    /* ... of four blocks at a time: a token's scale and sums of one block are
+     * 4 and 32 bytes of a 128-byte line that its other blocks share, and
+     * fetched block by block they were a quarter of the lines a workgroup asked
+     * the L2 for (Q4_K gate + up, 3001 tokens: 92.5M against 77.5M requests; the
+     * FFN's projections 2096 against 2060 us) */
+    auto fetch_side = [&](int b0) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int b = min(b0 + k, B - 1);
+            sc4[k] = scales[sc_at + b];
+            if constexpr (kHasMin<TYPE>)
+                sums4[k] = *reinterpret_cast<const u32x4 *>(sums + (gs_at + b) * 16 + 8 * (tid & 1));
+        }
     };
+    auto of4 = [](auto x0, auto x1, auto x2, auto x3, int k) { return k < 2 ? (k == 0 ? x0 : x1) : (k == 2 ? x2 : x3); };
 
     f32x4 total[kTiles]; /* tile i: tokens 16 i .. of the wave's 16 rows */
 #pragma unroll
     for (int i = 0; i < kTiles; ++i) total[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     fetch_acts(0, 0);
-    fetch_regs(0);
+    fetch_weights(0);
+    fetch_side(0);
     for (int b = 0; b < B; ++b) {
-        const int buf = b & 1;
-        if (tid < NT) ascale[buf][tid] = my_scale;
+        const int buf = b & 1, k4 = b & 3;
+        if (tid < NT) ascale[buf][tid] = of4(sc4[0], sc4[1], sc4[2], sc4[3], k4);
         if constexpr (kHasMin<TYPE>) {
             f16x8 g8;
 #pragma unroll
-            for (int k = 0; k < 8; ++k)
-                g8[k] = (_Float16)(float)(int)(int16_t)((my_sums[k >> 1] >> (16 * (k & 1))) & 0xffffu);
+            for (int k = 0; k < 8; ++k) {
+                const int w = k >> 1;
+                const uint32_t v = of4(sums4[0][w], sums4[1][w], sums4[2][w], sums4[3][w], k4);
+                g8[k] = (_Float16)(float)(int)(int16_t)((v >> (16 * (k & 1))) & 0xffffu);
+            }
             if (tid < 2 * NT) *reinterpret_cast<f16x8 *>(&gsum[buf][tid >> 1][8 * (tid & 1)]) = g8;
         }
         /* this block's activations have landed (every wave's share), and every
@@ -1791,7 +1805,8 @@ Q38_DEV void gemm_wide_q8k(const q38_gemv_args &a) {
         const float sb = kHasMin<TYPE> ? __uint_as_float((__float_as_uint(d) & ~hbm) | (__float_as_uint(dmin) & hbm)) : d;
         if (b + 1 < B) {
             fetch_acts(b + 1, buf ^ 1);
-            fetch_regs(b + 1);
+            fetch_weights(b + 1);
+            if (k4 == 3) fetch_side(b + 1);
         }
         __builtin_amdgcn_sched_barrier(0);
 
