@@ -1242,76 +1242,6 @@ Q38_DEV uint32_t fold_weights(uint32_t q, int sc) {
     }
 }
 
-/* The byte planes of the lane's 16 scaled weights of k step st: bh alone,
- * bh and bl, or (Q5_K) bh, bl and bx; bm the bytes of the second sum. */
-template <int TYPE>
-Q38_DEV void gemm_step_planes(const Unit<TYPE> &u, const UnitScales<TYPE> &s, uint32_t hm, const uint8_t *grid, int st,
-                              i32x4 &bh, i32x4 &bl, i32x4 &bx, i32x4 &bm) {
-    auto word = [&](int k) { return kGemmHalfUnit<TYPE> ? u.w[k] : (u.w[k] & ~hm) | (u.w[k + 4] & hm); };
-    if constexpr (TYPE == Q38_GGML_Q4_K) {
-        /* w = sc q with sc = 8 sh + sl: the planes q sh and q sl
-         * (at most 15 x 7 = 105 per byte) are packed 16-bit
-         * products of the quant bytes, no carry between bytes */
-        const unsigned short sh = (unsigned short)(s.sc[st] >> 3), sl = (unsigned short)(s.sc[st] & 7);
-        const u16x2 SH = {sh, sh}, SL = {sl, sl};
-        const int c = st >> 1, nib = st & 1;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const u16x2 q = __builtin_bit_cast(u16x2, (word(4 + 8 * c + j) >> (4 * nib)) & 0x0F0F0F0Fu);
-            bh[j] = __builtin_bit_cast(int, q * SH);
-            bl[j] = __builtin_bit_cast(int, q * SL);
-            bm[j] = s.mn[st] * 0x01010101;
-        }
-    } else if constexpr (TYPE == Q38_GGML_Q5_K) {
-        /* w = sc q, q <= 31: three planes of sc = 16 s2 + 4 s1 +
-         * s0 (each at most 3, q s <= 93 per byte) */
-        const unsigned short s2 = (unsigned short)(s.sc[st] >> 4), s1 = (unsigned short)((s.sc[st] >> 2) & 3),
-                             s0 = (unsigned short)(s.sc[st] & 3);
-        const u16x2 S2 = {s2, s2}, S1 = {s1, s1}, S0 = {s0, s0};
-        const int c = st >> 1, nib = st & 1;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t qv = ((word(12 + 8 * c + j) >> (4 * nib)) & 0x0F0F0F0Fu) |
-                                (((word(4 + j) >> st) & 0x01010101u) << 4);
-            const u16x2 q = __builtin_bit_cast(u16x2, qv);
-            bh[j] = __builtin_bit_cast(int, q * S2);
-            bl[j] = __builtin_bit_cast(int, q * S1);
-            bx[j] = __builtin_bit_cast(int, q * S0);
-            bm[j] = s.mn[st] * 0x01010101;
-        }
-    } else if constexpr (TYPE == Q38_GGML_Q6_K) {
-        const int sc = (int)(((uint32_t)s.sc[2 * st] & ~hm) | ((uint32_t)s.sc[2 * st + 1] & hm));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int hf = st >> 2, kq = st & 3;
-            const uint32_t ql = word(16 * hf + 8 * (kq & 1) + j);
-            const uint32_t qh = word(32 + 8 * hf + j);
-            const uint32_t q = ((ql >> (4 * (kq >> 1))) & 0x0F0F0F0Fu) | (((qh >> (2 * kq)) & 0x03030303u) << 4);
-            uint32_t hi, lo;
-            split_weights(q, sc, (short)32, hi, lo);
-            bh[j] = (int)hi;
-            bl[j] = (int)lo;
-        }
-    } else {
-        uint32_t q[4], second[4];
-        int sc;
-        short off;
-        gemm_step_bytes<TYPE>(u, s, st, hm, grid, q, sc, off, second);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            if constexpr (kGemmPlanes<TYPE> == 1) {
-                bh[j] = (int)fold_weights<TYPE>(q[j], sc);
-            } else {
-                uint32_t hi, lo;
-                split_weights(q[j], sc, off, hi, lo);
-                bh[j] = (int)hi;
-                bl[j] = (int)lo;
-            }
-            bm[j] = (int)second[j];
-        }
-    }
-}
-
 /* One block's f32 terms for a tile of 32 tokens x 32 rows (the lane's 16
  * outputs: row l % 32, tokens 8J + 4(l/32) + i for element 4J + i): the
  * integer sums on the matrix unit, then the reference's f32 block term.
@@ -1321,11 +1251,73 @@ Q38_DEV void gemm_step_planes(const Unit<TYPE> &u, const UnitScales<TYPE> &s, ui
 template <int TYPE, typename AOf, typename AsOf, typename Sink>
 Q38_DEV void gemm_tile_terms(const Unit<TYPE> &u, const UnitScales<TYPE> &s, uint32_t hm, const uint8_t *grid,
                              AOf A_of, AsOf as_of, Sink sink) {
+    auto word = [&](int k) { return kGemmHalfUnit<TYPE> ? u.w[k] : (u.w[k] & ~hm) | (u.w[k + 4] & hm); };
     i32x16 wsum = i32x16{}, lsum = i32x16{}, xsum = i32x16{}, msum = i32x16{};
 #pragma unroll
     for (int st = 0; st < 8; ++st) {
         i32x4 bh, bl, bx, bm;
-        gemm_step_planes<TYPE>(u, s, hm, grid, st, bh, bl, bx, bm);
+        if constexpr (TYPE == Q38_GGML_Q4_K) {
+            /* w = sc q with sc = 8 sh + sl: the planes q sh and q sl
+             * (at most 15 x 7 = 105 per byte) are packed 16-bit
+             * products of the quant bytes, no carry between bytes */
+            const unsigned short sh = (unsigned short)(s.sc[st] >> 3), sl = (unsigned short)(s.sc[st] & 7);
+            const u16x2 SH = {sh, sh}, SL = {sl, sl};
+            const int c = st >> 1, nib = st & 1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const u16x2 q = __builtin_bit_cast(u16x2, (word(4 + 8 * c + j) >> (4 * nib)) & 0x0F0F0F0Fu);
+                bh[j] = __builtin_bit_cast(int, q * SH);
+                bl[j] = __builtin_bit_cast(int, q * SL);
+                bm[j] = s.mn[st] * 0x01010101;
+            }
+        } else if constexpr (TYPE == Q38_GGML_Q5_K) {
+            /* w = sc q, q <= 31: three planes of sc = 16 s2 + 4 s1 +
+             * s0 (each at most 3, q s <= 93 per byte) */
+            const unsigned short s2 = (unsigned short)(s.sc[st] >> 4), s1 = (unsigned short)((s.sc[st] >> 2) & 3),
+                                 s0 = (unsigned short)(s.sc[st] & 3);
+            const u16x2 S2 = {s2, s2}, S1 = {s1, s1}, S0 = {s0, s0};
+            const int c = st >> 1, nib = st & 1;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t qv = ((word(12 + 8 * c + j) >> (4 * nib)) & 0x0F0F0F0Fu) |
+                                    (((word(4 + j) >> st) & 0x01010101u) << 4);
+                const u16x2 q = __builtin_bit_cast(u16x2, qv);
+                bh[j] = __builtin_bit_cast(int, q * S2);
+                bl[j] = __builtin_bit_cast(int, q * S1);
+                bx[j] = __builtin_bit_cast(int, q * S0);
+                bm[j] = s.mn[st] * 0x01010101;
+            }
+        } else if constexpr (TYPE == Q38_GGML_Q6_K) {
+            const int sc = (int)(((uint32_t)s.sc[2 * st] & ~hm) | ((uint32_t)s.sc[2 * st + 1] & hm));
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int hf = st >> 2, kq = st & 3;
+                const uint32_t ql = word(16 * hf + 8 * (kq & 1) + j);
+                const uint32_t qh = word(32 + 8 * hf + j);
+                const uint32_t q = ((ql >> (4 * (kq >> 1))) & 0x0F0F0F0Fu) | (((qh >> (2 * kq)) & 0x03030303u) << 4);
+                uint32_t hi, lo;
+                split_weights(q, sc, (short)32, hi, lo);
+                bh[j] = (int)hi;
+                bl[j] = (int)lo;
+            }
+        } else {
+            uint32_t q[4], second[4];
+            int sc;
+            short off;
+            gemm_step_bytes<TYPE>(u, s, st, hm, grid, q, sc, off, second);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (kGemmPlanes<TYPE> == 1) {
+                    bh[j] = (int)fold_weights<TYPE>(q[j], sc);
+                } else {
+                    uint32_t hi, lo;
+                    split_weights(q[j], sc, off, hi, lo);
+                    bh[j] = (int)hi;
+                    bl[j] = (int)lo;
+                }
+                bm[j] = (int)second[j];
+            }
+        }
         const i32x4 A = A_of(st);
         wsum = mfma_i8(A, bh, wsum);
         if constexpr (kGemmPlanes<TYPE> >= 2) lsum = mfma_i8(A, bl, lsum);
@@ -1377,7 +1369,7 @@ Q38_DEV void gemm_q8k(const q38_gemv_args &a) {
     const int rows = a.rows[0];
     const int row = blockIdx.x * kGemmRows + wave * 32 + (lane & 31);
     const int rowc = min(row, rows - 1);
-    const int t0 = a.tok_begin + blockIdx.y * kGemmTokens;
+    const int t0 = (int)(blockIdx.y + (uint32_t)a.tok_begin / kGemmTokens) * kGemmTokens;
     const int T = a.n_tokens;
     const int8_t *quants = static_cast<const int8_t *>(a.q8k);
     const int16_t *sums = reinterpret_cast<const int16_t *>(quants + (size_t)T * width);
@@ -1652,13 +1644,18 @@ Q38_DEV void part_planes(const Part<TYPE> &u, uint32_t hbm, uint32_t hm, const u
         unit_scales<TYPE>(u.u, s);
 #pragma unroll
         for (int p = 0; p < 4; ++p) {
-            i32x4 h0, l0, x0, m0, h1, l1, x1, m1;
-            gemm_step_planes<TYPE>(u.u, s, hm, grid, p, h0, l0, x0, m0);
-            gemm_step_planes<TYPE>(u.u, s, hm, grid, 4 + p, h1, l1, x1, m1);
+            uint32_t q0[4], q1[4], unused[4];
+            int sc0, sc1;
+            short off; /* the same for every step */
+            gemm_step_bytes<TYPE>(u.u, s, p, hm, grid, q0, sc0, off, unused);
+            gemm_step_bytes<TYPE>(u.u, s, 4 + p, hm, grid, q1, sc1, off, unused);
+            const int sc = (int)pick((uint32_t)sc0, (uint32_t)sc1);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                bh[p][j] = (int)pick((uint32_t)h0[j], (uint32_t)h1[j]);
-                if constexpr (kGemmPlanes<TYPE> >= 2) bl[p][j] = (int)pick((uint32_t)l0[j], (uint32_t)l1[j]);
+                uint32_t hi, lo;
+                split_weights(pick(q0[j], q1[j]), sc, off, hi, lo);
+                bh[p][j] = (int)hi;
+                bl[p][j] = (int)lo;
             }
         }
         d = s.d;
