@@ -192,6 +192,13 @@ def test_linear_core_decode_matches_reference(ctx, ref, synth, margin):
     check_state(margin, d_delta.download(), s_ref)
 
 
+@pytest.mark.parametrize("T", [320, 321, 512, 513])
+def test_gdn_chunked_prefill_prep_parts(ctx, ref, synth, margin, T):
+    """5, 6, 8 and 9 chunks: the prep's three value heads over three
+    workgroups, two (one of them with a single head) and one."""
+    test_gdn_chunked_prefill_matches_reference(ctx, ref, synth, margin, T)
+
+
 @pytest.mark.parametrize("T", [5, 40, 70, 200])
 def test_linear_core_prefill_matches_reference(ctx, ref, synth, margin, T):
     """batch_linear_attention's token loop (ops.rs:1088-1099) in one call."""
