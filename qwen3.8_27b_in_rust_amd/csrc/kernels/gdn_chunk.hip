@@ -18,7 +18,7 @@
  * Every decay factor is exp of a difference G_t - G_s (s <= t) or of G_t
  * itself, never exp(-G), so nothing overflows when decays are strong.
  *
- * q38_gdn_chunk_prep (grid (16 q/k heads, chunks, sequences)) computes W, U',
+ * q38_gdn_chunk_prep (grid (16 q/k heads x parts, chunks, sequences)) computes W, U',
  * Bm and G of every chunk in parallel, for the 3 value heads that read one
  * q/k head; T comes from a blocked inverse in f32 (16x16 diagonal blocks by
  * substitution, the off-diagonal blocks by T_ij = -T_ii sum_k A_ik T_kj on
