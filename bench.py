@@ -914,7 +914,9 @@ F32_PATH_TYPES = {0: ("F32", 4.0), 1: ("F16", 2.0), 30: ("BF16", 2.0), 8: ("Q8_0
 def _f32_path_kernels(ty: int) -> list:
     """The kernels q38_gemv_f32 may launch for weight type ty."""
     sfx = F32_PATH_TYPES[ty][0].lower()
-    kerns = ["q38_gemm_f32_" + sfx, "q38_gemm_f32s_" + sfx] + (["q38_gemm_f32w_" + sfx] if ty != 0 else [])
+    kerns = ["q38_gemm_f32_" + sfx, "q38_gemm_f32s_" + sfx, "q38_gemm_f32s8_" + sfx]
+    kerns += ["q38_gemm_f32sr_" + sfx] if ty in (0, 1) else []
+    kerns += ["q38_gemm_f32w_" + sfx] if ty != 0 else []
     if ty == 8:
         return kerns + ["q38_gemv_f32_q8_0s_r2_t1", "q38_gemv_f32_q8_0s_r2_t2", "q38_gemv_f32_q8_0s_r2_t4",
                         "q38_gemv_f32_q8_0s_r4_t8"]

@@ -170,6 +170,8 @@ struct q38_ctx {
     hipFunction_t f_gemv_f32[3] = {nullptr, nullptr, nullptr}; /* F32, F16, BF16 weights */
     hipFunction_t f_gemm_f32[4] = {nullptr, nullptr, nullptr, nullptr}; /* the same, on the matrix unit */
     hipFunction_t f_gemm_f32s[4] = {nullptr, nullptr, nullptr, nullptr}; /* few tokens, k split over the waves */
+    hipFunction_t f_gemm_f32sr[2] = {nullptr, nullptr}; /* ... past one workgroup per CU (F32, F16) */
+    hipFunction_t f_gemm_f32s8[4] = {nullptr, nullptr, nullptr, nullptr}; /* ... on 8 waves, half the rows */
     hipFunction_t f_gemm_f32w[4] = {nullptr, nullptr, nullptr, nullptr}; /* 128-token tiles (not F32) */
     hipFunction_t f_gemv_q80s[4] = {}; /* Q8_0, activations staged in LDS: TP 1, 2, 4 (RW 2), 8 (RW 4) */
     hipModule_t mod_synth = nullptr;
@@ -454,6 +456,12 @@ int q38_ctx_create(q38_ctx **out, int device, const char *module_dir) {
     Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32s[1], ctx->mod_proj, "q38_gemm_f32s_f16"));
     Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32s[2], ctx->mod_proj, "q38_gemm_f32s_bf16"));
     Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32s[3], ctx->mod_proj, "q38_gemm_f32s_q8_0"));
+    Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32sr[0], ctx->mod_proj, "q38_gemm_f32sr_f32"));
+    Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32sr[1], ctx->mod_proj, "q38_gemm_f32sr_f16"));
+    Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32s8[0], ctx->mod_proj, "q38_gemm_f32s8_f32"));
+    Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32s8[1], ctx->mod_proj, "q38_gemm_f32s8_f16"));
+    Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32s8[2], ctx->mod_proj, "q38_gemm_f32s8_bf16"));
+    Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32s8[3], ctx->mod_proj, "q38_gemm_f32s8_q8_0"));
     Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32w[1], ctx->mod_proj, "q38_gemm_f32w_f16"));
     Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32w[2], ctx->mod_proj, "q38_gemm_f32w_bf16"));
     Q38_HIP(hipModuleGetFunction(&ctx->f_gemm_f32w[3], ctx->mod_proj, "q38_gemm_f32w_q8_0"));
@@ -665,6 +673,12 @@ int q38_kernel_timer_start(q38_ctx *ctx, const char *kernel_name, int max_launch
     else if (name == "q38_gemm_f32s_f16") f = ctx->f_gemm_f32s[1];
     else if (name == "q38_gemm_f32s_bf16") f = ctx->f_gemm_f32s[2];
     else if (name == "q38_gemm_f32s_q8_0") f = ctx->f_gemm_f32s[3];
+    else if (name == "q38_gemm_f32sr_f32") f = ctx->f_gemm_f32sr[0];
+    else if (name == "q38_gemm_f32sr_f16") f = ctx->f_gemm_f32sr[1];
+    else if (name == "q38_gemm_f32s8_f32") f = ctx->f_gemm_f32s8[0];
+    else if (name == "q38_gemm_f32s8_f16") f = ctx->f_gemm_f32s8[1];
+    else if (name == "q38_gemm_f32s8_bf16") f = ctx->f_gemm_f32s8[2];
+    else if (name == "q38_gemm_f32s8_q8_0") f = ctx->f_gemm_f32s8[3];
     else if (name == "q38_gemm_f32w_f16") f = ctx->f_gemm_f32w[1];
     else if (name == "q38_gemm_f32w_bf16") f = ctx->f_gemm_f32w[2];
     else if (name == "q38_gemm_f32w_q8_0") f = ctx->f_gemm_f32w[3];
@@ -2266,13 +2280,14 @@ int q38_gemv_f32(q38_ctx *ctx, int ggml_type, int rows, int width, const void *d
     const long tok_groups = ((long)n_tokens + Q38_GEMV_TOKENS - 1) / Q38_GEMV_TOKENS;
     if (row_groups > 0x7FFFFFFFL || tok_groups > 65535) return fail("too many rows or tokens");
     /* Widths a multiple of 64 take the bf16 matrix unit from 4 tokens on
-     * (Q8_0: from 9, its staged GEMV being faster up to 8): up to 32 tokens,
-     * or where the 128 x 64 tiles would give fewer than half a workgroup per
-     * CU, 64 rows x 32 tokens per workgroup with k split over its waves;
-     * otherwise the 128 x 64 tiles (measured on 48-17408 rows x 5120 and
-     * 5120 x 17408, 2-4096 tokens: e.g. BF16 17408 x 5120 at 15 tokens 72
-     * against 188 us as the GEMV, at 48 tokens 105 against 123 us on the
-     * split-k form; 48 x 5120 at 4096 tokens 39 against 99 us) */
+     * (Q8_0: from 9, its staged GEMV being faster up to 8), few rows aside
+     * (below): up to 32 tokens, or where the 128 x 64 tiles would give fewer
+     * than half a workgroup per CU, a split-k form, 64 or 32 rows x 32 tokens
+     * per workgroup with k split over its waves; otherwise the 128 x 64 tiles
+     * (measured on 48-17408 rows x 5120 and 5120 x 17408, 2-4096 tokens: e.g.
+     * BF16 17408 x 5120 at 15 tokens 72 against 188 us as the GEMV, at 48
+     * tokens 105 against 123 us on the split-k form; 48 x 5120 at 4096 tokens
+     * 39 against 99 us) */
     const bool unit_width = width % Q38_GEMM_F32_K == 0;
     const long big_wgs = ((long)rows + Q38_GEMM_F32_ROWS - 1) / Q38_GEMM_F32_ROWS *
                          (((long)n_tokens + Q38_GEMM_F32_TOKENS - 1) / Q38_GEMM_F32_TOKENS);
@@ -2291,23 +2306,33 @@ int q38_gemv_f32(q38_ctx *ctx, int ggml_type, int rows, int width, const void *d
         s.n_tokens = n_tokens;
         /* Few rows (the 48-row beta / alpha projections) are too few tiles for
          * the matrix unit to beat the GEMV's row per wave, whose loads are
-         * contiguous, while that grid is at most two workgroups per CU: 48 x
-         * 5120 F32 at 4 / 32 / 331 tokens 9.3 / 15.3 / 27.9 us against 28 / 40 /
-         * 40 (78.7 against 41.5 at 1024), BF16 9.9 / 15.9 / 28.6 against 18 / 30 /
-         * 30; 1024 x 5120 F32 at 16 tokens 16.9 against 33 (BF16 at 32: 32.9
-         * against 30.4) */
-        if (ti < 3 && row_groups * tok_groups <= 2L * ctx->cu_count) {
-            s.form = Q38_F32S_ROWS;
-            return ctx->launch(ctx->f_gemm_f32s[ti], (unsigned)row_groups, (unsigned)tok_groups, 1, 256, &s);
-        }
+         * contiguous, while that grid is at most two workgroups per CU (48 x
+         * 5120, the GEMV against the 8-wave form, us: F32 at 4 / 32 / 331
+         * tokens 8.5 / 14.4 / 27.1 against 27.2 / 39.2 / 39.7, BF16 9.2 / 15.1 /
+         * 28.3 against 17.3 / 29.4 / 29.7, and past the line, at 500, 30.7
+         * against 29.5; 1024 x 5120 at 16 F32 17.4 against 33.2, BF16 16.7
+         * against 22.8).  Rows that one 32-row tile holds, in 16 bits, leave it
+         * earlier, from 1.5 workgroups per CU on inputs past 4M values: each
+         * pass of 8 tokens reads its input again for 4 rows only (16 x 5120
+         * BF16 at 1000 tokens 29.5 against 26.7, F32 28.2 against 33.8; 4 x
+         * 17408 BF16 at 4096 127.9 against 76.5) */
+        const long row_wgs = row_groups * tok_groups;
+        const bool one_tile = ti > 0 && rows <= 32 && 2 * row_wgs > 3L * ctx->cu_count &&
+                              (long)n_tokens * width > (1L << 22);
+        if (ti < 3 && row_wgs <= 2L * ctx->cu_count && !one_tile)
+            return ctx->launch(ctx->f_gemv_f32[ti], (unsigned)row_groups, (unsigned)tok_groups, 1, 256, &s);
         /* 64 rows a workgroup, or, where that leaves half the CUs without one,
-         * 32 rows on twice the waves */
+         * 32 rows on twice the waves (48 x 5120 F32 at 32 tokens 39.2 against
+         * 50.2 us, 1024 x 5120 BF16 at 32 29.7 against 38.4; no shape of 1-4096
+         * rows and 4-4096 tokens more than 4% the other way) */
         const long toks = ((long)n_tokens + 31) / 32;
-        const bool few = 2 * (((long)rows + 63) / 64 * toks) <= (long)ctx->cu_count;
-        const int tile_rows = few ? 32 : 64;
-        s.form = few ? Q38_F32S_8_WAVES : Q38_F32S_4_WAVES;
-        return ctx->launch(ctx->f_gemm_f32s[ti], (unsigned)((rows + tile_rows - 1) / tile_rows), (unsigned)toks, 1,
-                           few ? 512 : 256, &s);
+        if (2 * (((long)rows + 63) / 64 * toks) <= (long)ctx->cu_count)
+            return ctx->launch(ctx->f_gemm_f32s8[ti], (unsigned)((rows + 31) / 32), (unsigned)toks, 1, 512, &s);
+        /* past one workgroup per CU the rolled loop (gemm_f32s), F16 from two
+         * token tiles on */
+        const bool rolled = ((long)rows + 63) / 64 * toks > (long)ctx->cu_count && (ti == 0 || (ti == 1 && toks > 1));
+        return ctx->launch(rolled ? ctx->f_gemm_f32sr[ti] : ctx->f_gemm_f32s[ti], (unsigned)((rows + 63) / 64),
+                           (unsigned)toks, 1, 256, &s);
     }
     q38_gemv_f32_args a;
     memset(&a, 0, sizeof(a));

@@ -2593,7 +2593,8 @@ Q38_GEMM_F32(q8_0, Q38_GGML_Q8_0)
  * the next slice's loads go out before this slice's matrix steps.  The four
  * waves' accumulators are added through LDS in wave order, so the sums do
  * not depend on timing.  grid (ceil(rows / 64), ceil(T / 32)), 256 threads;
- * width a multiple of 64.
+ * width a multiple of 64.  q38_gemm_f32s8_* is the same over 32 rows on 8 waves,
+ * with more slices in flight.
  */
 template <int TYPE> struct F32sRaw { u32x4 v[TYPE == Q38_GGML_F32 ? 4 : 2]; };
 template <> struct F32sRaw<Q38_GGML_Q8_0> { u32x4 v[1]; uint32_t tail, d; };
@@ -2660,12 +2661,21 @@ Q38_DEV void f32s_parts(const F32sRaw<TYPE> &r, int sb, const uint8_t *p, u32x4 
 }
 
 /* RT row tiles of 32 per workgroup, k split over W waves, DEPTH 32-wide slices
- * of k in flight per wave.  Two instances: (2, 4, 1), and where that grid
- * leaves half the CUs idle or more (1, 8, 4).  Bound by the CU's load path: a
- * lane's 16-byte pieces lie a row apart, and few rows are few CUs -- 48 x 5120
- * F32 at 32 tokens, one workgroup, 50 us; on the second form 40. */
-template <int TYPE, int RT, int W, int DEPTH>
-Q38_DEV void gemm_f32s_tile(const q38_gemv_f32_args &a, float *red) {
+ * of k in flight per wave.  Bound by the CU's load path: a lane's 16-byte pieces
+ * lie a row apart, and few rows are few CUs.  Three instances, each a kernel of
+ * its own: (1, 8, 4) where 64-row workgroups would leave half the CUs idle or
+ * more; (2, 4, 1); and on larger grids of F32 and F16 weights the same ROLLED, a
+ * slice loaded at its loop's head and moved down at its end.  The unrolled loop
+ * waits for a load only where it is used, which pays while a workgroup has the
+ * CU to itself (10240 rows at 9 tokens, us unrolled / rolled: x 17408 F32 172 /
+ * 198, Q8_0 105 / 134, x 5120 F16 35.3 / 42.5); with two on some CUs it is the
+ * slower (17408 x 17408 F32 at 4 tokens 373 / 346; 10240 x 17408 F16 at 40 238 /
+ * 223), F16 up to 32 tokens aside (17408 x 5120 at 32 81 / 85).  BF16 and Q8_0
+ * gain from it on every grid (BF16 17408 x 5120 at 9 tokens 59.2 / 62.3), Q8_0
+ * scheduled for two waves a SIMD (10240 x 5120 at 9 33.8 against 35.8). */
+template <int TYPE, int RT, int W, int DEPTH, bool ROLLED>
+Q38_DEV void gemm_f32s(const q38_gemv_f32_args &a) {
+    __shared__ float red[(W - 1) * RT * 16 * 64];
     constexpr int PW = F32wParts<TYPE>::n;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -2695,45 +2705,62 @@ Q38_DEV void gemm_f32s_tile(const q38_gemv_f32_args &a, float *red) {
     for (int r = 0; r < RT; ++r)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[r][e] = 0.0f;
+    /* slice sl, held in entry k */
+    auto compute = [&](int sl, int k) {
+        f32x16 blk[RT];
+        if constexpr (TYPE == Q38_GGML_Q8_0) {
 #pragma unroll
-    for (int k = 0; k < DEPTH; ++k)
-        if (s_begin + k < s_end) load(s_begin + k, k);
-    for (int s0 = s_begin; s0 < s_end; s0 += DEPTH + 1) {
+            for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int k = 0; k <= DEPTH; ++k) {
-            const int sl = s0 + k;
-            if (sl >= s_end) break;
-            if (sl + DEPTH < s_end) load(sl + DEPTH, (k + DEPTH) % (DEPTH + 1));
-            f32x16 blk[RT];
-            if constexpr (TYPE == Q38_GGML_Q8_0) {
+                for (int e = 0; e < 16; ++e) blk[r][e] = 0.0f;
+        }
 #pragma unroll
-                for (int r = 0; r < RT; ++r)
+        for (int sb = 0; sb < 2; ++sb) {
+            float v[8];
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) blk[r][e] = 0.0f;
+            for (int i = 0; i < 8; ++i) v[i] = xs[k][2 * sb + (i >> 2)][i & 3];
+            u32x4 ax[3];
+            split_parts<3>(v, ax);
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                u32x4 bw[PW];
+                f32s_parts<TYPE>(ws[k][r], sb, wp[r] + (size_t)sl * 34 + 2 + 16 * h, bw);
+                if constexpr (TYPE == Q38_GGML_Q8_0) blk[r] = f32w_products<PW>(ax, bw, blk[r]);
+                else acc[r] = f32w_products<PW>(ax, bw, acc[r]);
             }
+        }
+        if constexpr (TYPE == Q38_GGML_Q8_0) {
 #pragma unroll
-            for (int sb = 0; sb < 2; ++sb) {
-                float v[8];
+            for (int r = 0; r < RT; ++r) {
+                /* this lane's output column is its own row l % 32 of tile r */
+                const float d = q38_f16(ws[k][r].d);
 #pragma unroll
-                for (int i = 0; i < 8; ++i) v[i] = xs[k][2 * sb + (i >> 2)][i & 3];
-                u32x4 ax[3];
-                split_parts<3>(v, ax);
-#pragma unroll
-                for (int r = 0; r < RT; ++r) {
-                    u32x4 bw[PW];
-                    f32s_parts<TYPE>(ws[k][r], sb, wp[r] + (size_t)sl * 34 + 2 + 16 * h, bw);
-                    if constexpr (TYPE == Q38_GGML_Q8_0) blk[r] = f32w_products<PW>(ax, bw, blk[r]);
-                    else acc[r] = f32w_products<PW>(ax, bw, acc[r]);
-                }
+                for (int e = 0; e < 16; ++e) acc[r][e] = __builtin_fmaf(d, blk[r][e], acc[r][e]);
             }
-            if constexpr (TYPE == Q38_GGML_Q8_0) {
+        }
+    };
+    if constexpr (ROLLED) {
+        static_assert(DEPTH == 1, "one slice ahead");
+        if (s_begin < s_end) load(s_begin, 0);
+        for (int sl = s_begin; sl < s_end; ++sl) {
+            if (sl + 1 < s_end) load(sl + 1, 1);
+            compute(sl, 0);
 #pragma unroll
-                for (int r = 0; r < RT; ++r) {
-                    /* this lane's output column is its own row l % 32 of tile r */
-                    const float d = q38_f16(ws[k][r].d);
+            for (int i = 0; i < 4; ++i) xs[0][i] = xs[1][i];
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) acc[r][e] = __builtin_fmaf(d, blk[r][e], acc[r][e]);
-                }
+            for (int r = 0; r < RT; ++r) ws[0][r] = ws[1][r];
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < DEPTH; ++k)
+            if (s_begin + k < s_end) load(s_begin + k, k);
+        for (int s0 = s_begin; s0 < s_end; s0 += DEPTH + 1) {
+#pragma unroll
+            for (int k = 0; k <= DEPTH; ++k) {
+                const int sl = s0 + k;
+                if (sl >= s_end) break;
+                if (sl + DEPTH < s_end) load(sl + DEPTH, (k + DEPTH) % (DEPTH + 1));
+                compute(sl, k);
             }
         }
     }
@@ -2761,23 +2788,20 @@ Q38_DEV void gemm_f32s_tile(const q38_gemv_f32_args &a, float *red) {
     }
 }
 
-template <int TYPE>
-Q38_DEV void gemm_f32s(const q38_gemv_f32_args &a) {
-    __shared__ float red[7 * 16 * 64];
-    static_assert(3 * 2 <= 7, "either form's partial sums");
-    if (a.form == Q38_F32S_8_WAVES) {
-        gemm_f32s_tile<TYPE, 1, 8, 4>(a, red);
-    } else if (a.form == Q38_F32S_ROWS) {
-        if constexpr (TYPE != Q38_GGML_Q8_0) gemv_f32<TYPE>(a); /* Q8_0 has no such launch */
-    } else {
-        gemm_f32s_tile<TYPE, 2, 4, 1>(a, red);
-    }
-}
-
-extern "C" __global__ __launch_bounds__(512) void q38_gemm_f32s_f32(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_F32>(a); }
-extern "C" __global__ __launch_bounds__(512) void q38_gemm_f32s_f16(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_F16>(a); }
-extern "C" __global__ __launch_bounds__(512) void q38_gemm_f32s_bf16(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_BF16>(a); }
-extern "C" __global__ __launch_bounds__(512) void q38_gemm_f32s_q8_0(q38_gemv_f32_args a) { gemm_f32s<Q38_GGML_Q8_0>(a); }
+#define Q38_GEMM_F32S(prefix, bounds, name, T, ...)                                                     \
+    extern "C" __global__ bounds void prefix##name(q38_gemv_f32_args a) { gemm_f32s<T, __VA_ARGS__>(a); }
+Q38_GEMM_F32S(q38_gemm_f32s_, __launch_bounds__(256), f32, Q38_GGML_F32, 2, 4, 1, false)
+Q38_GEMM_F32S(q38_gemm_f32s_, __launch_bounds__(256), f16, Q38_GGML_F16, 2, 4, 1, false)
+Q38_GEMM_F32S(q38_gemm_f32s_, __launch_bounds__(256), bf16, Q38_GGML_BF16, 2, 4, 1, false)
+Q38_GEMM_F32S(q38_gemm_f32s_, __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))), q8_0, Q38_GGML_Q8_0, 2, 4,
+              1, false)
+Q38_GEMM_F32S(q38_gemm_f32sr_, __launch_bounds__(256), f32, Q38_GGML_F32, 2, 4, 1, true)
+Q38_GEMM_F32S(q38_gemm_f32sr_, __launch_bounds__(256), f16, Q38_GGML_F16, 2, 4, 1, true)
+Q38_GEMM_F32S(q38_gemm_f32s8_, __launch_bounds__(512), f32, Q38_GGML_F32, 1, 8, 4, false)
+Q38_GEMM_F32S(q38_gemm_f32s8_, __launch_bounds__(512), f16, Q38_GGML_F16, 1, 8, 4, false)
+Q38_GEMM_F32S(q38_gemm_f32s8_, __launch_bounds__(512), bf16, Q38_GGML_BF16, 1, 8, 4, false)
+Q38_GEMM_F32S(q38_gemm_f32s8_, __launch_bounds__(512), q8_0, Q38_GGML_Q8_0, 1, 8, 4, false)
+#undef Q38_GEMM_F32S
 
 /*
  * Q8_0 weights below 16 tokens: a workgroup of 4 waves takes 4 RW rows (RW

@@ -385,13 +385,10 @@ typedef struct {
  * row; the bf16 matrix-unit forms (width a multiple of Q38_GEMM_F32_K):
  * q38_gemm_f32_*, grid (ceil(rows / Q38_GEMM_F32_ROWS), ceil(T /
  * Q38_GEMM_F32_TOKENS)), q38_gemm_f32w_*, the same with
- * Q38_GEMM_F32_WIDE_TOKENS tokens per workgroup, and q38_gemm_f32s_*, grid
- * (ceil(rows / 64), ceil(T / 32)), 256 threads. */
-/* q38_gemm_f32s_*: 64 rows x 32 tokens on 4 waves; 32 x 32 on 8 (512 threads);
- * or the GEMV's waves, a row and 8 tokens each, on the GEMV's grid */
-#define Q38_F32S_4_WAVES 0
-#define Q38_F32S_8_WAVES 1
-#define Q38_F32S_ROWS 2
+ * Q38_GEMM_F32_WIDE_TOKENS tokens per workgroup, and with k split
+ * over the waves q38_gemm_f32s_* and q38_gemm_f32sr_*, grid (ceil(rows / 64),
+ * ceil(T / 32)), 256 threads, and q38_gemm_f32s8_*, grid (ceil(rows / 32), ceil(T / 32)), 512
+ * threads. */
 #define Q38_GEMM_F32_ROWS 128
 #define Q38_GEMM_F32_TOKENS 64
 #define Q38_GEMM_F32_WIDE_TOKENS 128
@@ -407,7 +404,7 @@ typedef struct {
     int32_t rows;
     int32_t width;
     int32_t n_tokens;
-    int32_t form; /* q38_gemm_f32s_*: Q38_F32S_* */
+    int32_t pad_;
 } q38_gemv_f32_args;
 
 /* Merge of split-K partials.  grid (n_seq, 24, 4). */

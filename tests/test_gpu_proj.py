@@ -321,7 +321,39 @@ def test_wide_tiles_bit_exact(ctx, ref, name, rows, T, kern):
 F32_PATH_SHAPES = [(48, HIDDEN, 1), (48, HIDDEN, 3), (257, 1024, 9), (5, 6144, 17), (1031, 2048, 1),
                    (48, HIDDEN, 64), (300, 1024, 100), (129, 768, 33), (64, 320, 16), (40, 1032, 20), (37, 64, 5),
                    (19, 17408, 2), (70, 14528, 3), (33, 6144, 15), (2048, 256, 512), (100, 1024, 9),
-                   (70, 17408, 12), (4100, 128, 4096)]
+                   (70, 17408, 12), (4100, 128, 4096),
+                   # 4-wave split k: 10 slices, partial row and token tiles; 2 slices, two waves without one
+                   (8300, 320, 16), (8300, 320, 33), (8300, 64, 32), (16400, 320, 16), (16400, 64, 32),
+                   (8300, 64, 40), (10300, 320, 40),
+                   # 8-wave: 8 slices a wave (its ring of 5 refilled twice), 1 or 2 a wave, 6 slices over 8 waves
+                   (330, 2048, 100), (1100, 448, 40), (1100, 192, 40),
+                   # both sides of the lines between the forms
+                   (2048, 256, 8), (2049, 256, 8), (8192, 64, 16), (8193, 64, 16),
+                   (16384, 64, 16), (16385, 64, 16), (16, HIDDEN, 824), (16, HIDDEN, 816)]
+
+
+def _f32_path_kernel(ctx, ty, rows, W, T):
+    """The kernel of a gemv_f32 call: the GEMV where the width is no multiple
+    of 64, for few tokens (Q8_0: activations staged in LDS) and for few rows;
+    the split-k forms up to 32 tokens or on small grids; else the 128-row
+    tiles."""
+    sfx = {0: "f32", 1: "f16", 30: "bf16", 8: "q8_0"}[ty]
+    cus = ctx.info()["cu_count"]
+    if W % 64 or T < (9 if ty == 8 else 4):
+        tp = min(t for t in (1, 2, 4, 8) if t >= min(T, 8))
+        return "q38_gemv_f32_" + sfx + ("s_r%d_t%d" % (4 if tp == 8 else 2, tp) if ty == 8 else "")
+    if T > 32 and 2 * (-(-rows // 128) * -(-T // 64)) >= cus:
+        wide = ty != 0 and -(-rows // 128) * -(-T // 128) >= 4 * cus  # 128-token tiles (not F32)
+        return ("q38_gemm_f32w_" if wide else "q38_gemm_f32_") + sfx
+    row_wgs = -(-rows // 4) * -(-T // 8)
+    one_tile = ty != 0 and rows <= 32 and 2 * row_wgs > 3 * cus and T * W > 1 << 22
+    if ty != 8 and row_wgs <= 2 * cus and not one_tile:
+        return "q38_gemv_f32_" + sfx
+    wgs = -(-rows // 64) * -(-T // 32)  # of the 4-wave split-k forms
+    if 2 * wgs <= cus:
+        return "q38_gemm_f32s8_" + sfx
+    rolled = wgs > cus and (ty == 0 or (ty == 1 and T > 32))
+    return ("q38_gemm_f32sr_" if rolled else "q38_gemm_f32s_") + sfx
 
 
 @pytest.mark.parametrize("name,rows,W,T", [(n, r, w, t) for n in sorted(F32_TYPES) for r, w, t in F32_PATH_SHAPES
@@ -329,24 +361,15 @@ F32_PATH_SHAPES = [(48, HIDDEN, 1), (48, HIDDEN, 3), (257, 1024, 9), (5, 6144, 1
 def test_gemv_f32_path(ctx, ref, margin, name, rows, W, T):
     """tensor_gemv_f32 / tensor_gemm_f32 for the weight types project()
     does not quantise for (the 48-row beta / alpha projections of a DeltaNet
-    layer and other shapes; several token passes; from 4 tokens on the
-    matrix-unit forms, with partial row and token tiles and k ranges that
-    leave a wave empty, and the GEMV where the width is not a multiple of
-    64): every element within 1e-5 of the
+    layer and other shapes; several token passes; every form the library
+    chooses from, on both sides of the lines between them, with partial row
+    and token tiles and k ranges that leave a wave empty): every element
+    within 1e-5 of the
     sum of |w x| of the oracle's sequential chain, and of the float64 dot of
     the weights decoded in numpy; a one-hot input row gives each weight
     exactly."""
     ty = F32_TYPES[name]
-    sfx = {0: "f32", 1: "f16", 30: "bf16", 8: "q8_0"}[ty]
-    if W % 64 or T < (9 if ty == 8 else 4):  # the GEMV; Q8_0: activations staged in LDS
-        tp = min(t for t in (1, 2, 4, 8) if t >= min(T, 8))
-        kern = "q38_gemv_f32_" + sfx + ("s_r%d_t%d" % (4 if tp == 8 else 2, tp) if ty == 8 else "")
-    else:  # the matrix unit: k split over the waves up to 32 tokens or on small grids
-        cus = ctx.info()["cu_count"]
-        big_wgs = -(-rows // 128) * -(-T // 64)
-        skinny = T <= 32 or 2 * big_wgs < cus
-        wide = ty != 0 and -(-rows // 128) * -(-T // 128) >= 4 * cus  # 128-token tiles (not F32)
-        kern = ("q38_gemm_f32s_" if skinny else "q38_gemm_f32w_" if wide else "q38_gemm_f32_") + sfx
+    kern = _f32_path_kernel(ctx, ty, rows, W, T)
     rng = np.random.default_rng(0x51333940 + ty + rows)
     x = rng.standard_normal((T, W)).astype(np.float32)
     if T > 1:

@@ -73,10 +73,19 @@ def test_split_block_gemm_fits_its_workgroups(kernels):
 
 
 def test_f32_path_kernels_do_not_spill(kernels):
-    """The f32-input path: the GEMV and the bf16 matrix-unit form (two
+    """The f32-input path: the GEMV and the bf16 matrix-unit forms (two
     workgroups per CU: at most 256 registers), no spills."""
     f32 = {k: v for k, v in kernels.items()
-           if k.startswith(("q38_gemv_f32_", "q38_gemm_f32_", "q38_gemm_f32s_", "q38_gemm_f32w_"))}
-    assert len(f32) == 18
+           if k.startswith(("q38_gemv_f32_", "q38_gemm_f32_", "q38_gemm_f32s_", "q38_gemm_f32sr_", "q38_gemm_f32s8_",
+                            "q38_gemm_f32w_"))}
+    assert len(f32) == 24
     for name, (vgpr, scratch) in f32.items():
         assert scratch == 0 and vgpr <= 256, (name, vgpr, scratch)
+
+
+def test_rolled_split_k_keeps_its_occupancy(kernels):
+    """The split-k form of grids past one workgroup per CU hides its loads
+    behind three waves a SIMD (168 registers), F16 four (128)."""
+    for name, limit in (("f32", 168), ("f16", 128)):
+        vgpr, _ = kernels["q38_gemm_f32sr_" + name]
+        assert vgpr <= limit, (name, vgpr, limit)
