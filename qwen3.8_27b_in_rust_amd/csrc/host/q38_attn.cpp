@@ -103,23 +103,23 @@ struct GemvType {
     const char *gemm_wide_kernel;
     int terms;
     int grid_bytes;
-    double wide_round; /* gemm_wide_toks */
+    double wide_round, tile_start; /* gemm_wide_toks */
 };
 constexpr GemvType kGemv[] = {
-    {Q38_GGML_Q4_K, "q38_gemv_q8k_q4k", "q38_gemm_q8k_q4k", "q38_gemm_ks_q8k_q4k", "q38_gemm_ks16_q8k_q4k", "q38_gemm_ks4_q8k_q4k", "q38_gemm_wide_q8k_q4k", 1, 0, 3.0},
-    {Q38_GGML_Q5_K, "q38_gemv_q8k_q5k", "q38_gemm_q8k_q5k", "q38_gemm_ks_q8k_q5k", "q38_gemm_ks16_q8k_q5k", "q38_gemm_ks4_q8k_q5k", "q38_gemm_wide_q8k_q5k", 1, 0, 2.5},
-    {Q38_GGML_Q6_K, "q38_gemv_q8k_q6k", "q38_gemm_q8k_q6k", "q38_gemm_ks_q8k_q6k", "q38_gemm_ks16_q8k_q6k", "q38_gemm_ks4_q8k_q6k", "q38_gemm_wide_q8k_q6k", 1, 0, 2.7},
-    {Q38_GGML_Q3_K, "q38_gemv_q8k_q3k", "q38_gemm_q8k_q3k", "q38_gemm_ks_q8k_q3k", "q38_gemm_ks16_q8k_q3k", "q38_gemm_ks4_q8k_q3k", "q38_gemm_wide_q8k_q3k", 1, 0, 3.2},
-    {Q38_GGML_IQ4_XS, "q38_gemv_q8k_iq4xs", "q38_gemm_q8k_iq4xs", "q38_gemm_ks_q8k_iq4xs", "q38_gemm_ks16_q8k_iq4xs", "q38_gemm_ks4_q8k_iq4xs", "q38_gemm_wide_q8k_iq4xs", 1, 0, 2.4},
-    {Q38_GGML_Q2_K, "q38_gemv_q8k_q2k", "q38_gemm_q8k_q2k", "q38_gemm_ks_q8k_q2k", "q38_gemm_ks16_q8k_q2k", "q38_gemm_ks4_q8k_q2k", "q38_gemm_wide_q8k_q2k", 1, 0, 3.2},
-    {Q38_GGML_IQ4_NL, "q38_gemv_q8k_iq4nl", "q38_gemm_q8k_iq4nl", nullptr, nullptr, nullptr, nullptr, 8, 0, 0.0},
-    {Q38_GGML_IQ2_XXS, "q38_gemv_q8k_iq2xxs", "q38_gemm_q8k_iq2xxs", "q38_gemm_ks_q8k_iq2xxs", "q38_gemm_ks16_q8k_iq2xxs", "q38_gemm_ks4_q8k_iq2xxs", "q38_gemm_wide_q8k_iq2xxs", 1, 256 * 8, 3.4},
-    {Q38_GGML_IQ2_XS, "q38_gemv_q8k_iq2xs", "q38_gemm_q8k_iq2xs", "q38_gemm_ks_q8k_iq2xs", "q38_gemm_ks16_q8k_iq2xs", "q38_gemm_ks4_q8k_iq2xs", "q38_gemm_wide_q8k_iq2xs", 1, 512 * 8, 3.4},
-    {Q38_GGML_IQ2_S, "q38_gemv_q8k_iq2s", "q38_gemm_q8k_iq2s", "q38_gemm_ks_q8k_iq2s", "q38_gemm_ks16_q8k_iq2s", "q38_gemm_ks4_q8k_iq2s", "q38_gemm_wide_q8k_iq2s", 1, 1024 * 8, 3.2},
-    {Q38_GGML_IQ3_XXS, "q38_gemv_q8k_iq3xxs", "q38_gemm_q8k_iq3xxs", "q38_gemm_ks_q8k_iq3xxs", "q38_gemm_ks16_q8k_iq3xxs", "q38_gemm_ks4_q8k_iq3xxs", "q38_gemm_wide_q8k_iq3xxs", 1, 256 * 4, 3.4},
-    {Q38_GGML_IQ3_S, "q38_gemv_q8k_iq3s", "q38_gemm_q8k_iq3s", "q38_gemm_ks_q8k_iq3s", "q38_gemm_ks16_q8k_iq3s", "q38_gemm_ks4_q8k_iq3s", "q38_gemm_wide_q8k_iq3s", 1, 512 * 4, 3.3},
-    {Q38_GGML_IQ1_S, "q38_gemv_q8k_iq1s", "q38_gemm_q8k_iq1s", "q38_gemm_ks_q8k_iq1s", "q38_gemm_ks16_q8k_iq1s", "q38_gemm_ks4_q8k_iq1s", nullptr, 1, 2048 * 8, 0.0},
-    {Q38_GGML_IQ1_M, "q38_gemv_q8k_iq1m", "q38_gemm_q8k_iq1m", "q38_gemm_ks_q8k_iq1m", "q38_gemm_ks16_q8k_iq1m", "q38_gemm_ks4_q8k_iq1m", nullptr, 1, 2048 * 8, 0.0},
+    {Q38_GGML_Q4_K, "q38_gemv_q8k_q4k", "q38_gemm_q8k_q4k", "q38_gemm_ks_q8k_q4k", "q38_gemm_ks16_q8k_q4k", "q38_gemm_ks4_q8k_q4k", "q38_gemm_wide_q8k_q4k", 1, 0, 2.85, 0.2},
+    {Q38_GGML_Q5_K, "q38_gemv_q8k_q5k", "q38_gemm_q8k_q5k", "q38_gemm_ks_q8k_q5k", "q38_gemm_ks16_q8k_q5k", "q38_gemm_ks4_q8k_q5k", "q38_gemm_wide_q8k_q5k", 1, 0, 2.5, 0.2},
+    {Q38_GGML_Q6_K, "q38_gemv_q8k_q6k", "q38_gemm_q8k_q6k", "q38_gemm_ks_q8k_q6k", "q38_gemm_ks16_q8k_q6k", "q38_gemm_ks4_q8k_q6k", "q38_gemm_wide_q8k_q6k", 1, 0, 2.85, 0.6},
+    {Q38_GGML_Q3_K, "q38_gemv_q8k_q3k", "q38_gemm_q8k_q3k", "q38_gemm_ks_q8k_q3k", "q38_gemm_ks16_q8k_q3k", "q38_gemm_ks4_q8k_q3k", "q38_gemm_wide_q8k_q3k", 1, 0, 3.35, 1.0},
+    {Q38_GGML_IQ4_XS, "q38_gemv_q8k_iq4xs", "q38_gemm_q8k_iq4xs", "q38_gemm_ks_q8k_iq4xs", "q38_gemm_ks16_q8k_iq4xs", "q38_gemm_ks4_q8k_iq4xs", "q38_gemm_wide_q8k_iq4xs", 1, 0, 2.55, 0.6},
+    {Q38_GGML_Q2_K, "q38_gemv_q8k_q2k", "q38_gemm_q8k_q2k", "q38_gemm_ks_q8k_q2k", "q38_gemm_ks16_q8k_q2k", "q38_gemm_ks4_q8k_q2k", "q38_gemm_wide_q8k_q2k", 1, 0, 3.35, 0.4},
+    {Q38_GGML_IQ4_NL, "q38_gemv_q8k_iq4nl", "q38_gemm_q8k_iq4nl", nullptr, nullptr, nullptr, nullptr, 8, 0, 0.0, 0.0},
+    {Q38_GGML_IQ2_XXS, "q38_gemv_q8k_iq2xxs", "q38_gemm_q8k_iq2xxs", "q38_gemm_ks_q8k_iq2xxs", "q38_gemm_ks16_q8k_iq2xxs", "q38_gemm_ks4_q8k_iq2xxs", "q38_gemm_wide_q8k_iq2xxs", 1, 256 * 8, 3.3, 0.6},
+    {Q38_GGML_IQ2_XS, "q38_gemv_q8k_iq2xs", "q38_gemm_q8k_iq2xs", "q38_gemm_ks_q8k_iq2xs", "q38_gemm_ks16_q8k_iq2xs", "q38_gemm_ks4_q8k_iq2xs", "q38_gemm_wide_q8k_iq2xs", 1, 512 * 8, 3.25, 0.6},
+    {Q38_GGML_IQ2_S, "q38_gemv_q8k_iq2s", "q38_gemm_q8k_iq2s", "q38_gemm_ks_q8k_iq2s", "q38_gemm_ks16_q8k_iq2s", "q38_gemm_ks4_q8k_iq2s", "q38_gemm_wide_q8k_iq2s", 1, 1024 * 8, 3.1, 0.6},
+    {Q38_GGML_IQ3_XXS, "q38_gemv_q8k_iq3xxs", "q38_gemm_q8k_iq3xxs", "q38_gemm_ks_q8k_iq3xxs", "q38_gemm_ks16_q8k_iq3xxs", "q38_gemm_ks4_q8k_iq3xxs", "q38_gemm_wide_q8k_iq3xxs", 1, 256 * 4, 3.3, 0.6},
+    {Q38_GGML_IQ3_S, "q38_gemv_q8k_iq3s", "q38_gemm_q8k_iq3s", "q38_gemm_ks_q8k_iq3s", "q38_gemm_ks16_q8k_iq3s", "q38_gemm_ks4_q8k_iq3s", "q38_gemm_wide_q8k_iq3s", 1, 512 * 4, 3.15, 0.6},
+    {Q38_GGML_IQ1_S, "q38_gemv_q8k_iq1s", "q38_gemm_q8k_iq1s", "q38_gemm_ks_q8k_iq1s", "q38_gemm_ks16_q8k_iq1s", "q38_gemm_ks4_q8k_iq1s", nullptr, 1, 2048 * 8, 0.0, 0.0},
+    {Q38_GGML_IQ1_M, "q38_gemv_q8k_iq1m", "q38_gemm_q8k_iq1m", "q38_gemm_ks_q8k_iq1m", "q38_gemm_ks16_q8k_iq1m", "q38_gemm_ks4_q8k_iq1m", nullptr, 1, 2048 * 8, 0.0, 0.0},
 };
 constexpr int kGemvTypes = (int)(sizeof(kGemv) / sizeof(kGemv[0]));
 /* The split-block GEMM's grid: at least this many workgroups (fewer: the
@@ -165,7 +165,7 @@ struct q38_ctx {
     hipFunction_t f_gemm_ks[kGemvTypes] = {};   /* and its split-block form */
     hipFunction_t f_gemm_ks16[kGemvTypes] = {}; /* ... on 16 waves */
     hipFunction_t f_gemm_ks4[kGemvTypes] = {};  /* ... on 4 waves */
-    hipFunction_t f_gemm_wide[kGemvTypes] = {}; /* the 128-token tiles */
+    hipFunction_t f_gemm_wide[kGemvTypes] = {}; /* the 128 x 256 tiles */
     hipFunction_t f_gemv_q8k[kGemvTypes] = {}; /* by kGemv index */
     hipFunction_t f_gemv_f32[3] = {nullptr, nullptr, nullptr}; /* F32, F16, BF16 weights */
     hipFunction_t f_gemm_f32[4] = {nullptr, nullptr, nullptr, nullptr}; /* the same, on the matrix unit */
@@ -1974,26 +1974,54 @@ int q38_quantize_q8_k(q38_ctx *ctx, int n_tokens, int width, const float *d_x, v
     return ctx->launch(ctx->f_quantize_q8k, (width / Q38_Q8K_BLOCK + 15) / 16, n_tokens, 1, 256, &a);
 }
 
-/* How many of a call's first tokens take the 128 x 256 tiles (0: none).
- * One of them runs per CU, so their time goes by whole rounds of cu_count
- * tiles, while the 128 x 64 tiles, two or three per CU, go by their number;
- * a small launch adds half a round of its tiles for its start and end.  So as
- * many full rounds as pay go to the wide tiles and the remaining tokens to
- * the small ones.  round: a wide round's time in rounds of cu_count small
- * tiles, measured per format on 17408 x 5120 at 3840 tokens (8 wide rounds,
- * 31.9 small ones; Q4_K 815 against 1093 us, Q6_K 821 / 1218, Q5_K 865 /
- * 1393, IQ4_XS 779 / 1301, Q2_K 725 / 890, IQ2_S 1052 / 1314). */
-static int gemm_wide_toks(long row_tiles, int n_tokens, int cu_count, double round) {
+/* Whether tokens of one matrix go to the split-block form: a grid of at most
+ * kGemmKsMaxPerCu of its workgroups per CU. */
+static bool on_split_block(int rows, long toks, int cu_count, long *wgs) {
+    *wgs = ((long)rows + Q38_GEMM_KS_ROWS - 1) / Q38_GEMM_KS_ROWS * ((toks + Q38_GEMM_KS_TOKENS - 1) / Q38_GEMM_KS_TOKENS);
+    return *wgs <= kGemmKsMaxPerCu * (long)cu_count;
+}
+
+/* How many of a call's first tokens take the 128 x 256 tiles (0: none), by the
+ * time of what each split launches, in rounds of cu_count 128 x 64 tiles:
+ *  - the wide tiles, one per CU, whole rounds of wide_round each, all matrices
+ *    (row_tiles tiles of 128 rows) in one launch;
+ *  - the other tokens a launch per matrix: 128 x 64 tiles, whole rounds too
+ *    (5120 x 17408 Q4_K at 1..5 rounds 155 / 215 / 355 / 440 / 560 us) and
+ *    tile_start for the launch, a single round 0.3 more; or the split-block
+ *    form, 0.3 per workgroup and CU and 0.25.
+ * The wide tiles are taken where that is 2% less than without them.  The
+ * constants are fitted per format to every split of 17408 + 17408, 12288 and
+ * 10240 + 6144 rows x 5120, 5120 x 6144 and 5120 x 17408 at 69 lengths of
+ * 183-3300 tokens (3707 calls: 0.847 of the time without wide tiles over them,
+ * the best split of each 0.8445, none slower by 1%; priced by tile counts with
+ * one start for all launches, 0.87 and up to 9% slower: Q6_K 17408 + 17408 at
+ * 560 tokens 433 against 409 us, Q3_K 5120 x 6144 at 2000 213 against 199). */
+static int gemm_wide_toks(const int *rows, const bool *take, int n_mats, int n_tokens, int cu_count, double wide_round,
+                          double tile_start) {
     const long most = ((long)n_tokens + Q38_GEMM_WIDE_TOKENS - 1) / Q38_GEMM_WIDE_TOKENS;
+    long row_tiles = 0;
+    for (int i = 0; i < n_mats; ++i)
+        if (take[i]) row_tiles += ((long)rows[i] + Q38_GEMM_ROWS - 1) / Q38_GEMM_ROWS;
     if (row_tiles * most > 0x3FFFFFFFL) return 0;
-    double best = 0.0;
+    auto rounds = [&](long tiles) { return (double)((tiles + cu_count - 1) / cu_count); };
+    double without = 0.0, best = 0.0;
     long best_n = 0;
     for (long n = 0; n <= most; ++n) {
         const long rest = std::max(0L, n_tokens - n * Q38_GEMM_WIDE_TOKENS);
-        const long small = row_tiles * ((rest + Q38_GEMM_TOKENS - 1) / Q38_GEMM_TOKENS);
-        const double cost = round * (double)((row_tiles * n + cu_count - 1) / cu_count) +
-                            (small > 0 ? (double)small / cu_count + 0.5 : 0.0);
-        if (n == 0 || cost < best) {
+        double cost = wide_round * rounds(row_tiles * n);
+        for (int i = 0; i < n_mats && rest > 0; ++i) {
+            if (!take[i]) continue;
+            long ks;
+            if (on_split_block(rows[i], rest, cu_count, &ks)) {
+                cost += 0.3 * (double)ks / cu_count + 0.25;
+            } else {
+                const double full = rounds(((long)rows[i] + Q38_GEMM_ROWS - 1) / Q38_GEMM_ROWS *
+                                           ((rest + Q38_GEMM_TOKENS - 1) / Q38_GEMM_TOKENS));
+                cost += full + tile_start + (full == 1.0 ? 0.3 : 0.0);
+            }
+        }
+        if (n == 0) without = best = cost;
+        if (cost <= best && cost < 0.98 * without) {
             best = cost;
             best_n = n;
         }
@@ -2047,7 +2075,7 @@ static int gemv_q8k_multi(q38_ctx *ctx, int ggml_type, int n_mats, const int *ro
 
     /* Many tokens: the int8 matrix-unit forms.  A matrix whose split-block
      * grid (32 rows x 32 tokens per workgroup) would exceed kGemmKsMaxPerCu
-     * workgroups per CU takes the 128 x 64 tiles, a launch of its own; from
+     * workgroups per CU takes the 128-row tiles (gemm_wide_toks); from
      * Q38_GEMM_MIN_TOKENS tokens on, the others share one split-block launch
      * where their grids add up to at least kGemmKsMinTiles workgroups (on
      * fewer, e.g. 1024 x 5120 alone below 64 tokens, the GEMV is faster)
@@ -2057,15 +2085,15 @@ static int gemv_q8k_multi(q38_ctx *ctx, int ggml_type, int n_mats, const int *ro
      * 1.4-2x faster).  IQ4_NL, which has only the 128 x 64 form, takes it
      * from Q38_GEMM_IQ4NL_MIN_TOKENS tokens (half as many for 8192+ rows). */
     const int ti = ti_occ;
-    const long ks_tok_tiles = ((long)n_tokens + Q38_GEMM_KS_TOKENS - 1) / Q38_GEMM_KS_TOKENS;
     bool on_gemv[Q38_GEMV_MAX_MATS] = {}, on_big[Q38_GEMV_MAX_MATS] = {};
     bool any_gemm = false, ks_call = false;
     long ks_total = 0; /* workgroups of the shared split-block launch */
     for (int i = 0; i < n_mats; ++i) {
         if (rows[i] == 0) continue;
         if (ctx->f_gemm_ks[ti] != nullptr) {
-            const long ks_tiles = ((long)rows[i] + Q38_GEMM_KS_ROWS - 1) / Q38_GEMM_KS_ROWS * ks_tok_tiles;
-            on_big[i] = n_tokens >= Q38_GEMM_MIN_TOKENS && ks_tiles > kGemmKsMaxPerCu * (long)ctx->cu_count;
+            long ks_tiles;
+            const bool small = on_split_block(rows[i], n_tokens, ctx->cu_count, &ks_tiles);
+            on_big[i] = n_tokens >= Q38_GEMM_MIN_TOKENS && !small;
             if (!on_big[i]) ks_total += ks_tiles;
         } else if (has_gemm) {
             on_big[i] = n_tokens >= Q38_GEMM_IQ4NL_MIN_TOKENS ||
@@ -2133,12 +2161,10 @@ static int gemv_q8k_multi(q38_ctx *ctx, int ggml_type, int n_mats, const int *ro
     /* The tiled matrices' tokens, the first wide_toks of them on the 128 x 256
      * tiles (gemm_wide_toks) and the rest, per matrix, on the split-block form
      * or the 128 x 64 tiles by the rule above */
-    long wide_row_tiles = 0;
-    for (int i = 0; i < n_mats; ++i)
-        if (on_big[i]) wide_row_tiles += ((long)rows[i] + Q38_GEMM_ROWS - 1) / Q38_GEMM_ROWS;
-    const int wide_toks = ctx->f_gemm_wide[ti] != nullptr && wide_row_tiles > 0
-                              ? gemm_wide_toks(wide_row_tiles, n_tokens, ctx->cu_count, kGemv[ti].wide_round)
-                              : 0;
+    const int wide_toks =
+        ctx->f_gemm_wide[ti] != nullptr && std::count(on_big, on_big + n_mats, true) > 0
+            ? gemm_wide_toks(rows, on_big, n_mats, n_tokens, ctx->cu_count, kGemv[ti].wide_round, kGemv[ti].tile_start)
+            : 0;
     if (wide_toks > 0) {
         long row_tiles;
         q38_gemv_args g = gemm_args(on_big, Q38_GEMM_ROWS, 0, wide_toks, row_tiles);
@@ -2150,9 +2176,8 @@ static int gemv_q8k_multi(q38_ctx *ctx, int ggml_type, int n_mats, const int *ro
         bool only[Q38_GEMV_MAX_MATS] = {};
         only[i] = true;
         const int rest = n_tokens - wide_toks;
-        const long ks_tiles = ((long)rows[i] + Q38_GEMM_KS_ROWS - 1) / Q38_GEMM_KS_ROWS *
-                              (((long)rest + Q38_GEMM_KS_TOKENS - 1) / Q38_GEMM_KS_TOKENS);
-        if (ctx->f_gemm_ks[ti] != nullptr && ks_tiles <= kGemmKsMaxPerCu * (long)ctx->cu_count) {
+        long ks_tiles;
+        if (ctx->f_gemm_ks[ti] != nullptr && on_split_block(rows[i], rest, ctx->cu_count, &ks_tiles)) {
             if (launch_ks(only, wide_toks, n_tokens)) return -1;
             continue;
         }

@@ -318,6 +318,36 @@ def test_wide_tiles_bit_exact(ctx, ref, name, rows, T, kern):
         arr.free()
 
 
+@pytest.mark.parametrize("name,rows,T,wide", [
+    ("Q6_K", [17408, 17408], 560, False),  # 2 wide token tiles and a split-block launch per matrix: 433 against 409 us
+    ("Q3_K", [5120], 2000, False),         # a wide round and 320 small tiles, two rounds of them: 213 against 199
+    ("IQ3_XXS", [5120], 2000, False),
+    ("Q4_K", [5120], 1100, True),          # three rounds of 128 x 64 tiles against one of wide ones
+    ("Q4_K", [5120], 400, False),          # two against one
+])
+def test_wide_tiles_are_taken_where_they_pay(ctx, ref, name, rows, T, wide):
+    """The rule that gives tokens to the 128 x 256 tiles counts what is
+    launched: whole rounds of either tiles and a start for each matrix's
+    remaining tokens (shapes whose other split measured slower, 5120 and 6144
+    wide, on 256 CUs)."""
+    if ctx.info()["cu_count"] != 256:
+        pytest.skip("the rounds are those of 256 CUs")
+    ty, W = TYPES[name], 256
+    x = _activations(T, W, 0x51333C80 + T)
+    d_q = _quantize_on_device(ctx, x)
+    q8 = ref.quantize_q8_k(x)
+    wbs = [_random_kquant(ty, r, W, 0x51333C81 + ty + i) for i, r in enumerate(rows)]
+    d_ws = [ctx.array(wb, np.uint8) for wb in wbs]
+    d_os = [ctx.empty((T, r)) for r in rows]
+    assert _ran(ctx, "q38_gemm_wide_q8k_" + name.lower().replace("_", ""),
+                lambda: ctx.gemv_q8_k_multi(ty, rows, W, d_ws, d_q, T, d_os)) == wide
+    for wb, d_o in zip(wbs, d_os):
+        want = ref.gemv_q8_k(ty, wb, q8, T, W, threads=16)
+        assert np.array_equal(d_o.download().view(np.uint32), want.view(np.uint32))
+    for arr in [d_q, *d_ws, *d_os]:
+        arr.free()
+
+
 F32_PATH_SHAPES = [(48, HIDDEN, 1), (48, HIDDEN, 3), (257, 1024, 9), (5, 6144, 17), (1031, 2048, 1),
                    (48, HIDDEN, 64), (300, 1024, 100), (129, 768, 33), (64, 320, 16), (40, 1032, 20), (37, 64, 5),
                    (19, 17408, 2), (70, 14528, 3), (33, 6144, 15), (2048, 256, 512), (100, 1024, 9),
