@@ -286,7 +286,10 @@ Q38_DEV void decode_split(const q38_decode_args &a) {
     }
     if (kPre) {
         q38_rope_table(rope_cs[hw], li, pos, a.theta_scale);
-        __builtin_amdgcn_wave_barrier(); /* the lanes of a half-wave read each other's entries below */
+        /* the lanes of a half-wave read each other's entries below: LDS serves a
+         * wave in order, the fence keeps the compiler to it */
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
         if (forms) {
             q38_norm_rope8(px0, px1, pw0, pw1, li, rope_cs[hw]);
             const float unit = forms_key ? 1.0f : Q38_SCORE_LOG2;
