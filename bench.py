@@ -928,8 +928,8 @@ def f32_path(pkg, ctx, reps: int):
     (q38_gemv_f32: F32, F16, BF16, Q8_0) through 17408 x 5120 at 1, 16 and
     4096 tokens and the 48-row beta / alpha shape (48 x 5120) at 4096: kernel
     duration, the kernel the library chose (the GEMV for few tokens, the
-    bf16 matrix unit's split-k or 128 x 64 form), weight bytes per second and useful f32
-    operations per second (2 x rows x width x tokens; the matrix unit runs 3,
+    bf16 matrix unit's split-k forms or 128-row tiles), weight bytes per second
+    and useful f32 operations per second (2 x rows x width x tokens; the matrix unit runs 3,
     5 or 6 bf16 products per multiply for BF16/Q8_0, F16, F32 weights).
     Weights are random bytes (timing only)."""
     res = {}
@@ -962,32 +962,37 @@ def f32_path(pkg, ctx, reps: int):
 
 def _q8k_kernels(ty: int) -> tuple:
     """The kernels q38_gemv_q8_k may launch for weight type ty: the
-    split-block matrix-unit forms (16, 8, 4 waves), the 128 x 64 one, the
-    GEMV (IQ4_NL: the last two)."""
+    split-block matrix-unit forms (16, 8, 4 waves), the 128 x 64 tiles, the
+    128 x 256 tiles and the GEMV (IQ4_NL: the second tiles and the
+    split-block forms aside; IQ1: the 128 x 256 tiles aside)."""
     gemv = GEMV_KERNELS[ty]
-    kernels = (gemv.replace("q38_gemv_q8k_", "q38_gemm_ks16_q8k_"), gemv.replace("q38_gemv_q8k_", "q38_gemm_ks_q8k_"),
-               gemv.replace("q38_gemv_q8k_", "q38_gemm_ks4_q8k_"), gemv.replace("gemv", "gemm"), gemv)
-    return kernels if ty != 20 else kernels[3:]
+    forms = ("gemm",) if ty == 20 else ("gemm_ks16", "gemm_ks", "gemm_ks4", "gemm")
+    forms += () if ty in (19, 20, 29) else ("gemm_wide",)
+    return tuple(gemv.replace("q38_gemv_q8k_", f"q38_{f}_q8k_") for f in forms) + (gemv,)
 
 
 def _timed_q8k_kernel(ctx, ty, work, reps, max_launches):
-    """(kernel, total ms, launches) of the weight-type-ty projection kernel
-    that reps calls of work() launch (the first of _q8k_kernels(ty) that
-    runs)."""
+    """(kernels joined by " + ", total ms, launches) of the weight-type-ty
+    projection kernels that reps calls of work() launch: a call may give its
+    tokens to two forms."""
+    ran, ms, launches = [], 0.0, 0
     for kern in _q8k_kernels(ty):
         ctx.kernel_timer_start(kern, max_launches)
         for _ in range(reps):
             work()
         k_ms, k_n = ctx.kernel_timer_stop()
         if k_n > 0:
-            return kern, k_ms, k_n
-    raise RuntimeError(f"no projection kernel of type {ty} was launched")
+            ran.append(kern)
+            ms += k_ms
+            launches += k_n
+    if not ran:
+        raise RuntimeError(f"no projection kernel of type {ty} was launched")
+    return " + ".join(ran), ms, launches
 
 
 def _timed_projection(ctx, ty, rows, width, w, q, n_tokens, out, reps):
-    """Kernel time per call of one projection and the kernel that ran it:
-    the split-block matrix-unit form (16, 8 or 4 waves), the 128 x 64 one or
-    the GEMV, as the library chose for the shape."""
+    """Kernel time per call of one projection and the kernels that ran it,
+    as the library chose for the shape."""
     kern, k_ms, _ = _timed_q8k_kernel(ctx, ty, lambda: ctx.gemv_q8_k(ty, rows, width, w, q, n_tokens, out), reps,
                                       reps * 64)
     return kern, k_ms / reps
@@ -995,9 +1000,9 @@ def _timed_projection(ctx, ty, rows, width, w, q, n_tokens, out, reps):
 
 def projection_sweep(pkg, ctx, reps: int):
     """The FFN gate (17408 x 5120 Q4_K) and down (5120 x 17408 Q6_K)
-    projections at 1 to 4096 tokens: the kernel q38_gemv_q8_k chose (GEMV,
-    split-block matrix-unit form of 16 / 8 / 4 waves, 128 x 64 tiles), its
-    duration and its rate in weight bytes and int8 operations.  One matrix,
+    projections at 1 to 4096 tokens: the kernels q38_gemv_q8_k chose (GEMV,
+    split-block matrix-unit form of 16 / 8 / 4 waves, 128 x 64 or 128 x 256
+    tiles), their duration and rate in weight bytes and int8 operations.  One matrix,
     reused (cache-resident below ~200 MB); random weights (timing only)."""
     res = {}
     for ty, rows, width, label in ((12, 17408, 5120, "q4k_17408x5120"), (14, 5120, 17408, "q6k_5120x17408")):
