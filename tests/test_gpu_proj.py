@@ -191,9 +191,9 @@ def test_gemm_many_tokens_bit_exact(ctx, ref, name, rows, W, T):
     its grid has 64 to 1280 workgroups: on 16 waves up to 256 workgroups
     (1, 5, 9 and 20 blocks, so the last round is partial), on 8 beyond
     (8200 x 16 with 1 block, 4200 x 40 with 9); 4100 x 1000 (4128 such
-    workgroups) takes the 128-row x 64-token tiles, as IQ4_NL does from 32
-    tokens (16 for 8192+ rows); 130 x 1280 (5 workgroups) stays on the
-    GEMV."""
+    workgroups) takes the 128-row tiles, 256 or 64 tokens wide as the format's
+    times have it, and IQ4_NL the 64-token ones from 32 tokens (16 for 8192+
+    rows); 130 x 1280 (5 workgroups) stays on the GEMV."""
     ty = TYPES[name]
     x = _activations(T, W, 0x513338F0 + T + W)
     d_q = _quantize_on_device(ctx, x)
@@ -287,7 +287,8 @@ def test_multi_matrices_share_the_split_block_launch(ctx, ref, name):
 @pytest.mark.parametrize("name,rows,T,kern", [
     ("Q4_K", [16384], 513, "wide"),           # two full token tiles, one token left to the split-block form
     ("Q6_K", [16384 - 127], 500, "wide"),     # a ragged row tile, a ragged token tile, no rest
-    ("Q5_K", [12288, 1024, 4096], 511, "wide"),  # three matrices in a launch
+    ("Q5_K", [12288, 1024, 4096], 511, "wide"),  # two matrices in a launch, the small one split-block
+    ("Q5_K", [12288, 2688, 4000], 511, "wide"),  # three in a launch, the last with a ragged row tile
     ("Q2_K", [16384], 768, "wide"), ("Q3_K", [16300], 520, "wide"), ("IQ4_XS", [16384], 400, "wide"),
     ("IQ2_S", [16384], 512, "wide"), ("IQ3_S", [16384], 640, "wide"), ("IQ2_XXS", [16384], 512, "wide"),
     ("IQ2_XS", [16384], 512, "wide"), ("IQ3_XXS", [16384], 512, "wide"),
@@ -316,6 +317,59 @@ def test_wide_tiles_bit_exact(ctx, ref, name, rows, T, kern):
         assert np.array_equal(d_o.download().view(np.uint32), want.view(np.uint32)), r
     for arr in [d_q, *d_ws, *d_os]:
         arr.free()
+
+
+WIDE_TYPES = sorted(set(TYPES) - {"IQ4_NL", "IQ1_S", "IQ1_M"})
+
+
+@pytest.mark.parametrize("name,blocks", [("Q4_K", 5), ("Q4_K", 6), ("Q5_K", 8), ("Q5_K", 9), ("Q2_K", 5), ("Q2_K", 9),
+                                         ("Q6_K", 5), ("Q6_K", 8), ("Q3_K", 9), ("IQ4_XS", 6), ("IQ2_S", 9),
+                                         ("IQ3_S", 5), ("Q4_K", 20), ("Q6_K", 20), ("IQ2_XXS", 20)])
+def test_wide_tiles_many_blocks_bit_exact(ctx, ref, name, blocks):
+    """Rows of 5 and more blocks: both activation buffers used again and
+    again, the scales and group sums fetched four blocks at a time with a
+    partial last fetch (5, 6, 9 blocks) and without (8, 20: a 5120-wide row);
+    the last token tile holds 10 tokens.  Tokens so small that scale products
+    are subnormal or vanish, and large ones, are the oracle's bits too."""
+    ty, rows, T, W = TYPES[name], 5000, 1290, 256 * blocks
+    x = _activations(T, W, 0x51333D00 + blocks)
+    for t, e in ((3, -90), (4, -104), (5, -112), (300, -118), (1289, 60)):
+        x[t] *= np.float32(2.0) ** e
+    d_q = _quantize_on_device(ctx, x)
+    q8 = ref.quantize_q8_k(x)
+    wb = _random_kquant(ty, rows, W, 0x51333D01 + ty + blocks)
+    d_w, d_o = ctx.array(wb, np.uint8), ctx.empty((T, rows))
+    assert _ran(ctx, "q38_gemm_wide_q8k_" + name.lower().replace("_", ""),
+                lambda: ctx.gemv_q8_k(ty, rows, W, d_w, d_q, T, d_o))
+    got = d_o.download()
+    some = np.arange(rows) if blocks < 20 else np.r_[0:260, 2430:2580, 4870:5000]
+    want = ref.gemv_q8_k(ty, np.ascontiguousarray(wb.reshape(rows, -1)[some]), q8, T, W, threads=16)
+    got = np.ascontiguousarray(got[:, some])
+    bad = np.argwhere(got.view(np.uint32) != want.view(np.uint32).reshape(got.shape))
+    assert bad.size == 0, (len(bad), bad[:4])
+    for arr in (d_q, d_w, d_o):
+        arr.free()
+
+
+@pytest.mark.parametrize("name", WIDE_TYPES)
+def test_wide_tiles_and_the_small_ones_after_them(ctx, ref, name):
+    """608 tokens of 16384 rows: two wide token tiles and 96 tokens on the 128
+    x 64 tiles, a full and a partial one, counted from token 512; 120 tokens,
+    128 x 64 tiles only."""
+    ty, sfx, rows, W = TYPES[name], name.lower().replace("_", ""), 16380, 768
+    wb = _random_kquant(ty, rows, W, 0x51333E01 + ty)
+    d_w = ctx.array(wb, np.uint8)
+    for T, kerns in ((608, ("wide_", "")), (120, ("",))):
+        x = _activations(T, W, 0x51333E00 + T)
+        d_q, d_o = _quantize_on_device(ctx, x), ctx.empty((T, rows))
+        call = lambda: ctx.gemv_q8_k(ty, rows, W, d_w, d_q, T, d_o)
+        for k in ("wide_", ""):
+            assert _ran(ctx, "q38_gemm_" + k + "q8k_" + sfx, call) == (k in kerns), (T, k)
+        want = ref.gemv_q8_k(ty, wb, ref.quantize_q8_k(x), T, W, threads=16)
+        assert np.array_equal(d_o.download().view(np.uint32), want.view(np.uint32)), T
+        d_q.free()
+        d_o.free()
+    d_w.free()
 
 
 @pytest.mark.parametrize("name,rows,T,wide", [

@@ -72,6 +72,15 @@ def test_split_block_gemm_fits_its_workgroups(kernels):
         assert vgpr <= 128 and scratch <= 48, (name, vgpr, scratch)
 
 
+def test_wide_tiles_fit_their_workgroups(kernels):
+    """The 128 x 256 tiles run 512 threads, two waves a SIMD: 256 registers at
+    most, none spilled."""
+    wide = {k: v for k, v in kernels.items() if k.startswith("q38_gemm_wide_q8k_")}
+    assert len(wide) == 11
+    for name, (vgpr, scratch) in wide.items():
+        assert vgpr <= 256 and scratch == 0, (name, vgpr, scratch)
+
+
 def test_f32_path_kernels_do_not_spill(kernels):
     """The f32-input path: the GEMV and the bf16 matrix-unit forms (two
     workgroups per CU: at most 256 registers), no spills."""
