@@ -1811,8 +1811,8 @@ static int gdn_chunked(q38_ctx *ctx, int n_seq, int n_tokens, float *d_state, in
         a.n_chunks = std::min(Q38_GDN_STAGE_CHUNKS, n_chunks - c0);
         /* one workgroup fits a CU: split the 3 value heads of each while every
          * part still starts at once (5 chunks of one sequence in thirds, 8 in
-         * two): linear_core of 16 / 100 / 331 tokens 34.9 / 42.9 / 73.6 us
-         * against 55.1 / 63.4 / 83.4 undivided */
+         * two): linear_core of 16 / 100 / 331 tokens 34 / 41 / 72 us
+         * against 55 / 63 / 82 undivided */
         const long base = (long)Q38_LIN_QK_HEADS * a.n_chunks * n_seq;
         a.prep_parts = 3 * base <= (long)ctx->cu_count ? 3 : 2 * base <= (long)ctx->cu_count ? 2 : 1;
         if (ctx->launch(ctx->f_chunk_prep, Q38_LIN_QK_HEADS * a.prep_parts, a.n_chunks, n_seq, 512, &a)) return -1;

@@ -1418,14 +1418,14 @@ Q38_DEV void gemm_q8k(const q38_gemv_args &a) {
 }
 
 
-/* Long prompts: a workgroup of 8 waves owns 128 rows x NT tokens (256 or 128),
- * wave w the 16 rows 16 w .. + 15 and every token, as 16 x 16 tiles
+/* Long prompts: a workgroup of 8 waves owns 128 rows x 256 tokens, wave w the
+ * 16 rows 16 w .. + 15 and every token, as 16 x 16 tiles
  * (v_mfma_i32_16x16x64_i8).  A SIMD issues one vector or matrix instruction
  * about every 4 cycles, whichever of its waves it comes from, and the 128 x 64
  * tiles above spent 1.7 times the matrix unit's time issuing conversions and
  * block terms (17408 x 5120 Q4_K, 3001 tokens).  So this form is built to issue
  * fewer of them:
- *  - a block's weights become byte planes once for NT tokens, each lane
+ *  - a block's weights become byte planes once for 256 tokens, each lane
  *    reading and converting only its own 64 of the 256 (lane l: row l % 16;
  *    of the block, k half hb = (l / 16) % 2, and of each 32 values the 16 of
  *    half h = l / 32);
@@ -1442,14 +1442,15 @@ Q38_DEV void gemm_q8k(const q38_gemv_args &a) {
  *    whole KiB), and the 16 lanes that a 16-byte LDS read serves together (8
  *    of one k quarter, the other 8 tokens of the next) meet distinct banks --
  *    with hb in the chunk's top bit they met in pairs.
- * Measured: 17408 x 5120 at 3840 tokens Q4_K 815 us against 1093 on the 128 x
- * 64 tiles (840 against 626 TOPS), Q6_K 821 / 1218, Q5_K 865 / 1393, Q3_K 780
- * / 961, Q2_K 725 / 890, IQ4_XS 779 / 1301, IQ2_S 1052 / 1314, IQ3_S 1150 /
- * 1406.  Bound now by what the two waves of a SIMD issue: matrix unit busy
- * 47% of the cycles, vector issue 51%, 15% of them at once, at the 1.9 GHz
- * the part keeps under this load.  Measured and not kept: 32 x 32 tiles (half
- * the matrix instructions, no room for two tiles' accumulators: 5-25%
- * slower), a higher priority for one wave of each SIMD (no change).
+ * Measured: 17408 x 5120 at 3840 tokens, us here / on the 128 x 64 tiles: Q4_K
+ * 770 / 1065 (889 against 643 TOPS), Q6_K 812 / 1194, Q5_K 844 / 1346, Q3_K 738 /
+ * 927, Q2_K 619 / 793, IQ4_XS 756 / 1240, IQ2_XXS 990 / 1242, IQ2_XS 978 / 1246,
+ * IQ2_S 987 / 1330, IQ3_XXS 1057 / 1318, IQ3_S 1076 / 1429.  Bound now by what
+ * the two waves of a SIMD issue: matrix unit busy 47% of the cycles, vector
+ * issue 51%, 15% of them at once, at the 1.9 GHz the part keeps under this
+ * load (Q4_K).  Measured and not kept: 32 x 32 tiles (half the matrix
+ * instructions, no room for two tiles' accumulators: 5-25% slower), a higher
+ * priority for one wave of each SIMD (no change).
  * A launch holds up to Q38_GEMV_MAX_MATS matrices of one input (row tiles
  * wg_begin[m] ..), its tiles in bands of 8 row tiles walked along the tokens,
  * a contiguous stretch of them per XCD, so that the 32 workgroups an XCD runs
@@ -1465,7 +1466,7 @@ template <int TYPE> constexpr bool kHasMin =
 
 /* A lane's part of a block: 64 weights (values 128 hb + 32 p + 16 h .. + 15 for
  * p = 0..3) and their scales.  The formats of the largest files load just
- * that; the lattice formats load the block and pick (Whole). */
+ * that; the lattice formats load the block and pick. */
 template <int TYPE> struct Part {
     Unit<TYPE> u;
 };
@@ -1475,9 +1476,6 @@ template <> struct Part<Q38_GGML_Q6_K> { u32x4 ql[2], qh, sc; uint32_t dh; };
 template <> struct Part<Q38_GGML_Q2_K> { u32x4 sc, q; uint32_t dd; };
 template <> struct Part<Q38_GGML_Q3_K> { u32x4 high, q, sc; uint32_t dh; };
 template <> struct Part<Q38_GGML_IQ4_XS> { u32x4 q[4]; uint32_t w0, w1; };
-template <int TYPE> constexpr bool kWholePart =
-    !(TYPE == Q38_GGML_Q4_K || TYPE == Q38_GGML_Q5_K || TYPE == Q38_GGML_Q6_K || TYPE == Q38_GGML_Q2_K ||
-      TYPE == Q38_GGML_Q3_K || TYPE == Q38_GGML_IQ4_XS);
 
 /* 16 bytes at a dword boundary */
 Q38_DEV u32x4 load16_4aligned(const uint8_t *p) {
@@ -1672,8 +1670,9 @@ Q38_DEV void part_planes(const Part<TYPE> &u, uint32_t hbm, uint32_t hm, const u
     }
 }
 
-template <int TYPE, int NT>
+template <int TYPE>
 Q38_DEV void gemm_wide_q8k(const q38_gemv_args &a) {
+    constexpr int NT = Q38_GEMM_WIDE_TOKENS;
     constexpr int kTiles = NT / 16; /* 16 x 16 tiles of a wave */
     static_assert(TYPE != Q38_GGML_IQ1_S && TYPE != Q38_GGML_IQ1_M, "IQ1 takes the 128 x 64 tiles");
     __shared__ __align__(16) int8_t act[2][NT][256];
@@ -2161,7 +2160,7 @@ extern "C" __global__ __launch_bounds__(256) void q38_gemm_q8k_iq1s(q38_gemv_arg
 extern "C" __global__ __launch_bounds__(256) void q38_gemm_q8k_iq1m(q38_gemv_args a) { gemm_q8k<Q38_GGML_IQ1_M>(a); }
 #define Q38_GEMM_WIDE(name, T)                                                                                    \
     extern "C" __global__ __launch_bounds__(kWideThreads, 2) void q38_gemm_wide_q8k_##name(q38_gemv_args a) {      \
-        gemm_wide_q8k<T, Q38_GEMM_WIDE_TOKENS>(a);                                                                \
+        gemm_wide_q8k<T>(a);                                                                                      \
     }
 Q38_GEMM_WIDE(q4k, Q38_GGML_Q4_K)
 Q38_GEMM_WIDE(q5k, Q38_GGML_Q5_K)
